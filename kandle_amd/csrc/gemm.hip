@@ -40,65 +40,30 @@ __device__ __forceinline__ void store4(TO* C, int64_t off, const float (&v)[4], 
 }
 
 // =============================================================================================
-// MFMA tile kernel.  Workgroup tile (64 WTM) x (64 WTN), k-step KS, 4 waves in a 2 x 2 layout, each
-// wave (32 WTM) x (32 WTN) = WTM x WTN tiles of 32 x 32 (64 x 128 tiles: 8 waves in 2 x 4, each
-// 32 x 32; gemm_waves): 128 x 128 for large problems, smaller
-// tiles when 128-tiles would leave CUs idle.  The tile shape does not change any result: every
-// output element is summed over k in the same 16-wide MFMA steps, in the same order, whatever the
-// tile that holds it.  The product is formed as C^T = B A^T
-// so that each lane owns one m row and 4 consecutive n per register group: A-operand = B rows (n),
-// B-operand = A rows (m), both k-contiguous 16-byte LDS reads.  LDS double buffered; global loads are
-// raw buffer loads (rows past M / N and columns past the k range read as zero without a branch).
+// MFMA tile kernel: C = A B^T of K-contiguous rows, a workgroup per GM x GN output tile (and k range).
+// The product is formed as C^T = B A^T so that each lane owns one m row and 4 consecutive n per
+// register group: A-operand = B rows (n), B-operand = A rows (m), both k-contiguous 16-byte LDS
+// reads.  Every output is summed over k in the same 16-wide MFMA steps, in the same order, so the
+// tile that holds it does not change its bits.
 //
 // SPLIT: S workgroups share one output tile, each summing its K range (kchunk columns, a multiple
 // of 128) of the products into fp32 partials part[split][m][n] (row-major, leading dimension N);
 // gemm_splitk_reduce_kernel -- or a consumer such as kh_add_rms_norm -- then adds the S partials
 // in split order (deterministic whichever workgroup finished last) and applies the epilogue.
-// =============================================================================================
-constexpr int kGemmPrefetch = 3;        // k-steps of global loads in flight per workgroup
-// Split launches (short k ranges, 128 x 64 tiles): 2 steps in flight (C5 prefill, two runs: o_proj
-// 14.56 -> 14.12 us, down 15.25 -> 14.93 us; the unsplit qkv product is 0.5 us slower at 2).
-constexpr int kGemmSplitPrefetch = 2;
-constexpr int kGemmT128Min = 256;       // 128-tiles from this many tiles up
-constexpr int kGemmSplitTarget = 512;   // split K until about this many 64-tile workgroups
-// Tiles (64 WTM) x (64 WTN) of split launches and of products too small for 128 x 128 tiles.
-// C5 prefill, M = 512 (bench.py --only gemm, three runs): split launches with 128 x 64 tiles (one
-// workgroup per CU) against 64 x 64 (two per CU): o_proj 15.25 -> 14.56 us, down 16.83 -> 15.25 us;
-// the unsplit qkv and gate/up products are 0.5-1.5 us slower with 128 x 64 or 64 x 128 tiles, and
-// a k-step of 128 on the rectangular tiles needs 256 VGPRs + 90 AGPRs and is slower everywhere.
-constexpr int kGemmSplitWTM = 2, kGemmSplitWTN = 1;
-// Split launches with fp32 activations (two MFMAs per k-step) take 64 x 128 tiles: C5 o_proj
-// 17.9 -> 16.3 us, down 22.0 -> 19.4 us (64 x 64: 16.7 / 20.4; 128 x 128: 21.1 / 26.2).
-constexpr int kGemmSplitF32WTM = 1, kGemmSplitF32WTN = 2;
-constexpr int kGemmSmallWTM = 1, kGemmSmallWTN = 1;
-constexpr int kGemmRectKS = 64;         // k-step of 128 x 64 and 64 x 128 tiles
-constexpr int kMaxSplits = 8;
-// Waves per workgroup on 64 x 128 tiles: 2 x 4 waves of 32 x 32, two per SIMD, so that one wave's
-// LDS traffic (and with fp32 activations its hi / lo split of A) overlaps the other's MFMAs.  C5
-// prefill, alternating builds on one box: float32 activations 2.87-2.90 -> 2.75-2.77 ms (GEMMs
-// 77.3-78.0 -> 75.2-75.8 us per layer), bf16 2.363-2.367 -> 2.316-2.332 ms.  Other tiles keep four
-// waves of (32 WTM) x (32 WTN).  Each output's k-steps and their order are unchanged.
-constexpr int kGemmWaves64x128 = 8;
-template <int WTM, int WTN>
-constexpr int gemm_waves() { return WTM == 1 && WTN == 2 ? kGemmWaves64x128 : 4; }
-constexpr int g_tile(int wt) { return 64 * wt; }
-
-// PF: k-steps of prefetch in flight (register ring of PF stages; the loop is unrolled by PF so the
-// stage indices are compile-time).  Tiles are numbered column-major (all m tiles of one n tile in a
-// row) and, when the workgroup count is a multiple of 8, dealt to the 8 XCDs in contiguous ranges
-// (the hardware hands workgroup i to XCD i mod 8): each XCD then reads its own columns of B (the
-// weights) into its L2, and only A (the activations) is read by every XCD.
-// SWIGLU (bf16 output, no split): B's rows interleave the gate and up projections in blocks of 8
-// (rows 16i .. 16i + 7: gate rows 8i .. 8i + 7; rows 16i + 8 .. 16i + 15: the matching up rows), so
-// every lane holds each gate accumulator and its up partner, and the epilogue stores
+// SWIGLU (no split): B's rows interleave the gate and up projections in blocks of 8 (rows 16i ..
+// 16i + 7: gate rows 8i .. 8i + 7; rows 16i + 8 .. 16i + 15: the matching up rows), so every lane
+// holds each gate accumulator and its up partner, and the epilogue stores
 // C[m, f] = bf16(silu(bf16(gate)) * bf16(up)) over N / 2 features f -- the values the separate
 // GEMM (bf16 store) and silu*mul kernel produce, without the [M, N] intermediate.
-// QKNR (bf16, 64 x 128 tiles, no split): the QKV projection of a prefill, whose output columns are
-// head rows of 128 (the q heads, then the k heads, then the v heads).  The epilogue stages the
-// tile, rounded to bf16 as the plain GEMM stores it, in LDS and reads it back one head row per
-// group of 8 lanes -- qk_norm_rope_kernel's layout -- to apply qk-norm + RoPE to q and k rows with
-// the same arithmetic (qk_norm_rope_row) and write q rows to q_out and k / v rows into the KV cache,
-// so the [M, N] projection output is never written.
+// QKNR (no split): the QKV projection of a prefill, whose output columns are head rows of 128 (the
+// q heads, then the k heads, then the v heads).  The epilogue stages the tile, rounded to bf16 as
+// the plain GEMM stores it, in LDS and reads it back one head row per group of 8 lanes --
+// qk_norm_rope_kernel's layout -- to apply qk-norm + RoPE to q and k rows with the same arithmetic
+// (qk_norm_rope_row) and write q rows to q_out and k / v rows into the KV cache, so the [M, N]
+// projection output is never written.
+// =============================================================================================
+constexpr int kMaxSplits = 8;
+
 struct QknrArgs {
   const uint16_t* wq = nullptr;       // q_norm / k_norm weights [128], bf16
   const uint16_t* wk = nullptr;
@@ -117,236 +82,65 @@ struct QknrArgs {
   const float* rope_cs = nullptr;
 };
 
-// TA = float (fp32 activations, the reference's float32 arithmetic): A is read as fp32 and each
-// value a is split into bf16 hi = bf16(a) and lo = bf16(a - hi) (a - hi is exact in fp32) when the
-// tile is copied to LDS, as two planes; every k-step then runs two MFMAs into the same accumulator,
-// W * hi and W * lo.  The weights are exactly bf16, so each product is W * a up to the 2^-17
-// relative error of hi + lo, fp32 accumulate; the epilogues keep their fp32 values (no bf16
-// rounding of the SwiGLU operands or of the qk-norm + RoPE input) and store fp32.
-// LDS bytes of the k loop (two stages of the A planes and the B tile): two workgroups per CU when
-// they fit the CU's 160 KiB, else one.
-template <typename TA, int WTM, int WTN, int KS>
-constexpr int gemm_lds_bytes() {
-  return 2 * ((sizeof(TA) == 4 ? 2 : 1) * g_tile(WTM) + g_tile(WTN)) * (KS + 8) * 2;
-}
-template <typename TA, int WTM, int WTN, int KS>
-constexpr int gemm_min_blocks() {
-  return 2 * gemm_lds_bytes<TA, WTM, WTN, KS>() <= 160 * 1024 ? 2 : 1;
-}
-
-template <typename TO, int WTM, int WTN, int KS, bool SPLIT, int PF = 1, bool SWIGLU = false, bool QKNR = false,
-          typename TA = uint16_t, int NW = 4>
-__global__ __launch_bounds__(NW * 64, (gemm_min_blocks<TA, WTM, WTN, KS>())) void gemm_bf16_nt_kernel(
-    const TA* __restrict__ A, int64_t lda, const uint16_t* __restrict__ B, int64_t ldb, TO* C, int64_t ldc,
-    const TO* cin, int64_t ldcin, const TO* __restrict__ bias, int M, int N, int K, float alpha, float beta,
-    int tiles_n, int splits, int kchunk, float* __restrict__ part, QknrArgs qa) {
+// The QKNR epilogue of a GM x GN tile (m0, n0) of NW waves: acc[a][b] holds, per lane, output row
+// m0 + wm + 32b + r and columns n0 + wn + 32a + 8(j/4) + 4g + j%4 (r = lane & 31, g = lane >> 5).
+// smem: the k loop's LDS; the caller has passed a barrier since the loop's last LDS read.
+template <typename TA, int AM, int AN, int GM, int GN, int NW>
+__device__ __forceinline__ void gemm_qknr_store(const f32x16 (&acc)[AN][AM], uint16_t* smem, int m0, int n0, int wm,
+                                                int wn, int M, int N, const QknrArgs& qa) {
   constexpr bool AF = std::is_same<TA, float>::value;
-  constexpr int GM = g_tile(WTM), GN = g_tile(WTN);
-  // NW waves in a 2 x NW/2 layout, each (32 WTM) x (32 AN): AN = WTN with four waves, WTN / 2 with
-  // eight (two per SIMD).
-  constexpr int NT = NW * 64, NWN = NW / 2, AN = 4 * WTN / NW;
-  static_assert(NW == 4 || (NW == 8 && WTN % 2 == 0), "four waves, or eight on tiles of even WTN");
-  constexpr int STR = KS + 8;  // LDS row stride (elements): 16-byte aligned, breaks bank aliasing
-  constexpr int APL = AF ? 2 : 1;                  // A planes in LDS: bf16, or hi and lo
-  constexpr int ATILE = GM * STR, BTILE = GN * STR, ASTG = APL * ATILE;
-  constexpr int AE = 16 / (int)sizeof(TA);         // A elements per 16-byte chunk
-  constexpr int CPR = KS / 8;                      // 16-byte chunks per B row per k-step
-  constexpr int CPRA = KS / AE;                    // 16-byte chunks per A row per k-step
-  constexpr int CPTA = GM * CPRA / NT;             // chunks per thread per A tile
-  constexpr int CPTB = GN * CPR / NT;              // chunks per thread per B tile
-  constexpr int CPTM = CPTA > CPTB ? CPTA : CPTB;
-  __shared__ __attribute__((aligned(16))) uint16_t smem[2 * (ASTG + BTILE)];
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int r = lane & 31, g = lane >> 5;
-  int bid = blockIdx.x;
-  if (PF > 1 && (gridDim.x & 7) == 0) bid = (bid & 7) * (gridDim.x >> 3) + (bid >> 3);
-  const int tile = SPLIT ? bid / splits : bid;
-  const int split = SPLIT ? bid % splits : 0;
-  const int tiles_m = (M + GM - 1) / GM;
-  const int tm = PF > 1 ? tile % tiles_m : tile / tiles_n, tn = PF > 1 ? tile / tiles_m : tile % tiles_n;
-  const int m0 = tm * GM, n0 = tn * GN;
-  const int wm = (wave / NWN) * 32 * WTM, wn = (wave % NWN) * 32 * AN;
-  const int kbeg = split * kchunk, kend = min(K, kbeg + kchunk);
-
-  // Byte ranges of this tile's rows; a row past the matrix or a column past the range reads zero.
-  const int mrows = min(GM, M - m0), nrows = min(GN, N - n0);
-  const auto ra = make_rsrc(A + (int64_t)m0 * lda, (uint32_t)(((int64_t)(mrows - 1) * lda + K) * sizeof(TA)));
-  const auto rb = make_rsrc(B + (int64_t)n0 * ldb, (uint32_t)(((int64_t)(nrows - 1) * ldb + K) * 2));
-
-  // Staging: the A (B) tile is GM (GN) rows x KS k = GM * CPR chunks of 16 B, CPTA (CPTB) per
-  // thread, in PF register stages.
-  uint4 ast[PF][CPTA], bst[PF][CPTB];
-  // Byte offsets fit 32 bits (the launcher checks 128 rows of lda / ldb); columns past kend map to
-  // 0xffffffff, past the range, and read zero (K % 8 == 0, so a chunk is all in or all out).  The
-  // loads are branch-free, so the compiler's load counting stays exact across the prefetch ring.
-  auto load_tile = [&](int stg, int kt) {
-#pragma unroll
-    for (int i = 0; i < CPTM; ++i) {
-      const int id = tid + NT * i;
-      if (i < CPTA) {
-        const int row = id / CPRA, kc = kt + AE * (id % CPRA);
-        const uint32_t ao =
-            kc < kend ? ((uint32_t)row * (uint32_t)lda + (uint32_t)kc) * (uint32_t)sizeof(TA) : 0xffffffffu;
-        ast[stg][i < CPTA ? i : 0] = buf_load16(ra, ao);
-      }
-      if (i < CPTB) {
-        const int row = id / CPR, kc = kt + 8 * (id % CPR);
-        const bool in = kc < kend;
-        const uint32_t bo = in ? ((uint32_t)row * (uint32_t)ldb + (uint32_t)kc) * 2u : 0xffffffffu;
-        // B (the weights) with the non-temporal hint: C5 prefill 2.413-2.428 -> 2.396-2.402 ms
-        bst[stg][i < CPTB ? i : 0] = buf_load16_nt(rb, bo);
-      }
+  static_assert(GN % 128 == 0 && GM % (8 * NW) == 0, "whole head rows of 128");
+  // Staged row stride (elements of TA): 272 B (bf16) or 528 B (fp32), 16-byte aligned rows.
+  constexpr int TSTR = 128 + 16 / (int)sizeof(TA);
+  // The tile is staged as the plain GEMM would store it: rounded to bf16, or fp32 with fp32
+  // activations; one head row of 128 columns at a time.
+  TA* tile = reinterpret_cast<TA*>(smem);
+  // 8 elements of TA at p (16 or 32 bytes) <-> 8 floats
+  auto ld8 = [](const TA* p, float (&v)[8]) {
+    if constexpr (AF) {
+      const float4 x0 = reinterpret_cast<const float4*>(p)[0], x1 = reinterpret_cast<const float4*>(p)[1];
+      v[0] = x0.x; v[1] = x0.y; v[2] = x0.z; v[3] = x0.w; v[4] = x1.x; v[5] = x1.y; v[6] = x1.z; v[7] = x1.w;
+    } else {
+      unpack_bf16x8(*reinterpret_cast<const uint4*>(p), v);
     }
   };
-  auto store_tile = [&](int stg, int buf) {
-    uint16_t* as = smem + buf * (ASTG + BTILE);
-    uint16_t* bs = as + ASTG;
-#pragma unroll
-    for (int i = 0; i < CPTM; ++i) {
-      const int id = tid + NT * i;
-      if (i < CPTA) {
-        const int row = id / CPRA, kc = AE * (id % CPRA);
-        const uint4 v = ast[stg][i < CPTA ? i : 0];
-        if constexpr (AF) {
-          // four fp32 values -> bf16 hi (plane 0) and lo = bf16(a - hi) (plane 1)
-          const float f[4] = {__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)};
-          const uint32_t h01 = pack_bf16x2(f[0], f[1]), h23 = pack_bf16x2(f[2], f[3]);
-          const uint32_t l01 = pack_bf16x2(f[0] - lo_bf16(h01), f[1] - hi_bf16(h01));
-          const uint32_t l23 = pack_bf16x2(f[2] - lo_bf16(h23), f[3] - hi_bf16(h23));
-          *reinterpret_cast<uint2*>(as + row * STR + kc) = make_uint2(h01, h23);
-          *reinterpret_cast<uint2*>(as + ATILE + row * STR + kc) = make_uint2(l01, l23);
-        } else {
-          *reinterpret_cast<uint4*>(as + row * STR + kc) = v;
-        }
-      }
-      if (i < CPTB) {
-        const int row = id / CPR, kc = 8 * (id % CPR);
-        *reinterpret_cast<uint4*>(bs + row * STR + kc) = bst[stg][i < CPTB ? i : 0];
-      }
+  auto st8 = [](TA* p, const float (&v)[8]) {
+    if constexpr (AF) {
+      reinterpret_cast<float4*>(p)[0] = make_float4(v[0], v[1], v[2], v[3]);
+      reinterpret_cast<float4*>(p)[1] = make_float4(v[4], v[5], v[6], v[7]);
+    } else {
+      *reinterpret_cast<uint4*>(p) = pack_bf16x8(v);
     }
   };
-
-  f32x16 acc[AN][WTM];  // [n tile][m tile]
-#pragma unroll
-  for (int a = 0; a < AN; ++a)
-#pragma unroll
-    for (int b = 0; b < WTM; ++b)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) acc[a][b][j] = 0.f;
-
-  const int nk = kend > kbeg ? (kend - kbeg + KS - 1) / KS : 0;
-  // Step t is in LDS buffer t & 1 and, before that, in register stage t % PF.  Iteration t loads
-  // step t + PF into the stage step t has left, computes step t, then moves step t + 1 (loaded PF - 1
-  // iterations earlier) into the other LDS buffer.  Steps past the end load zeros and are stored
-  // into the idle buffer, so the main loop has no branches between a load and its use.
-  auto step = [&](int t, int u) {
-    load_tile(u, kbeg + (t + PF) * KS);
-    const uint16_t* as = smem + (t & 1) * (ASTG + BTILE);
-    const uint16_t* bs = as + ASTG;
-#pragma unroll
-    for (int kc = 0; kc < KS / 16; ++kc) {
-      bf16x8 av[APL][WTM], bv[AN];
-#pragma unroll
-      for (int pl = 0; pl < APL; ++pl)
-#pragma unroll
-        for (int i = 0; i < WTM; ++i)
-          av[pl][i] = as_bf16x8(
-              *reinterpret_cast<const uint4*>(as + pl * ATILE + (wm + 32 * i + r) * STR + 16 * kc + 8 * g));
-#pragma unroll
-      for (int i = 0; i < AN; ++i)
-        bv[i] = as_bf16x8(*reinterpret_cast<const uint4*>(bs + (wn + 32 * i + r) * STR + 16 * kc + 8 * g));
+  const int t8 = lane & 7, rs = lane >> 3;      // 8 lanes per head row, 8 rows per wave step
+  const bool cache_mode = qa.kv_cache_len > 0;
+#pragma unroll 1
+  for (int hh = 0; hh < GN / 128; ++hh) {
+    if (hh > 0) __syncthreads();
+    if (wn / 128 == hh) {
 #pragma unroll
       for (int a = 0; a < AN; ++a)
 #pragma unroll
-        for (int b = 0; b < WTM; ++b)
+        for (int b = 0; b < AM; ++b)
 #pragma unroll
-          for (int pl = 0; pl < APL; ++pl)
-            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bv[a], av[pl][b], acc[a][b], 0, 0, 0);
+          for (int q = 0; q < 4; ++q) {
+            TA* dst = tile + (wm + 32 * b + r) * TSTR + wn % 128 + 32 * a + 8 * q + 4 * g;
+            if constexpr (AF) {
+              *reinterpret_cast<float4*>(dst) =
+                  make_float4(acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]);
+            } else {
+              uint2 w;
+              w.x = pack_bf16x2(acc[a][b][4 * q], acc[a][b][4 * q + 1]);
+              w.y = pack_bf16x2(acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]);
+              *reinterpret_cast<uint2*>(dst) = w;
+            }
+          }
     }
-    store_tile((u + 1) % PF, (t + 1) & 1);
     __syncthreads();
-  };
-  if (nk > 0) {
-#pragma unroll
-    for (int s2 = 0; s2 < PF; ++s2) load_tile(s2, kbeg + s2 * KS);
-    store_tile(0, 0);
-    __syncthreads();
-    int t = 0;
-    for (; t + PF <= nk; t += PF) {
-#pragma unroll
-      for (int u = 0; u < PF; ++u) step(t + u, u);
-    }
-#pragma unroll
-    for (int u = 0; u + 1 < PF; ++u)
-      if (t + u < nk) step(t + u, u);
-  }
-
-  if constexpr (SPLIT) {
-    // Raw fp32 partial of this split: part[split][m][n] (N % 4 == 0, so four consecutive n of a
-    // register group are all in range or all out).
-    float* mine = part + (int64_t)split * M * N;
-#pragma unroll
-    for (int b = 0; b < WTM; ++b) {
-      const int m = m0 + wm + 32 * b + r;
-      if (m >= M) continue;
-#pragma unroll
-      for (int a = 0; a < AN; ++a)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int n = n0 + wn + 32 * a + 8 * q + 4 * g;
-          if (n >= N) continue;
-          *reinterpret_cast<float4*>(mine + (int64_t)m * N + n) =
-              make_float4(acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]);
-        }
-    }
-    return;
-  }
-
-  // Epilogue: acc[a][b] lane holds m = m0 + wm + 32b + r, n = n0 + wn + 32a + 8(j/4) + 4g + j%4.
-  if constexpr (QKNR) {
-    static_assert(sizeof(TO) == sizeof(TA) && WTM == 1 && WTN == 2 && !SPLIT && !SWIGLU,
-                  "QKNR: 64 x 128 tiles, output of the activations' type");
-    // Staged row stride (elements of TA): 272 B (bf16) or 528 B (fp32), 16-byte aligned rows.
-    constexpr int TSTR = 128 + 16 / (int)sizeof(TA);
-    static_assert(GM * TSTR * (int)sizeof(TA) <= 2 * (ASTG + BTILE) * 2, "the staged tile fits the k loop's LDS");
-    // Every wave has passed the k loop's last barrier: its LDS is free.  The tile is staged as the
-    // plain GEMM would store it: rounded to bf16, or fp32 with fp32 activations.
-    TA* tile = reinterpret_cast<TA*>(smem);
-#pragma unroll
-    for (int a = 0; a < AN; ++a)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        TA* dst = tile + (wm + r) * TSTR + wn + 32 * a + 8 * q + 4 * g;
-        if constexpr (AF) {
-          *reinterpret_cast<float4*>(dst) =
-              make_float4(acc[a][0][4 * q], acc[a][0][4 * q + 1], acc[a][0][4 * q + 2], acc[a][0][4 * q + 3]);
-        } else {
-          uint2 w;
-          w.x = pack_bf16x2(acc[a][0][4 * q], acc[a][0][4 * q + 1]);
-          w.y = pack_bf16x2(acc[a][0][4 * q + 2], acc[a][0][4 * q + 3]);
-          *reinterpret_cast<uint2*>(dst) = w;
-        }
-      }
-    __syncthreads();
-    // 8 elements of TA at p (16 or 32 bytes) <-> 8 floats
-    auto ld8 = [](const TA* p, float (&v)[8]) {
-      if constexpr (AF) {
-        const float4 x0 = reinterpret_cast<const float4*>(p)[0], x1 = reinterpret_cast<const float4*>(p)[1];
-        v[0] = x0.x; v[1] = x0.y; v[2] = x0.z; v[3] = x0.w; v[4] = x1.x; v[5] = x1.y; v[6] = x1.z; v[7] = x1.w;
-      } else {
-        unpack_bf16x8(*reinterpret_cast<const uint4*>(p), v);
-      }
-    };
-    auto st8 = [](TA* p, const float (&v)[8]) {
-      if constexpr (AF) {
-        reinterpret_cast<float4*>(p)[0] = make_float4(v[0], v[1], v[2], v[3]);
-        reinterpret_cast<float4*>(p)[1] = make_float4(v[4], v[5], v[6], v[7]);
-      } else {
-        *reinterpret_cast<uint4*>(p) = pack_bf16x8(v);
-      }
-    };
-    const int hd = n0 / 128;                      // q heads, then k heads, then v heads
-    const int t8 = lane & 7, rs = lane >> 3;      // 8 lanes per head row, 8 rows per wave step
+    const int hd = n0 / 128 + hh;               // q heads, then k heads, then v heads
+    if (hd * 128 >= N) continue;                // a tile column past the last head
     const bool is_q = hd < qa.hq, is_k = !is_q && hd < qa.hq + qa.hkv;
     float wa[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, wb[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     float f[8];
@@ -357,7 +151,6 @@ __global__ __launch_bounds__(NW * 64, (gemm_min_blocks<TA, WTM, WTN, KS>())) voi
 #pragma unroll
       for (int j = 0; j < 8; ++j) f[j] = qa.inv_freq[8 * t8 + j];
     }
-    const bool cache_mode = qa.kv_cache_len > 0;
 #pragma unroll
     for (int st = 0; st < GM / (8 * NW); ++st) {
       const int row = wave * (GM / NW) + st * 8 + rs;
@@ -400,52 +193,377 @@ __global__ __launch_bounds__(NW * 64, (gemm_min_blocks<TA, WTM, WTN, KS>())) voi
         st8(dst + 64 + 8 * t8, c8);
       }
     }
-    return;
   }
-  const bool vec = ((reinterpret_cast<uintptr_t>(C) & (4 * sizeof(TO) - 1)) == 0) && ((ldc & 3) == 0);
-  if constexpr (SWIGLU) {
-    // Register groups q = 0, 2 hold gate rows n0 + wn + 32a + 8q + 4g + e, q + 1 the up rows 8 later:
-    // feature f = (n0 + wn + 32a) / 2 + 4q + 4g + e (q = 0, 2).  N / 2 is a multiple of 8.
-    const int NH = N / 2;
+}
+
+// The other epilogues, wave by wave, each with its own WLDS bytes of LDS: a register group holds 16
+// bytes of a row, so stored as they are the 64 lanes write 32-byte pieces of 32 rows; instead the
+// finished blocks of 32 rows are turned in LDS and stored as whole row segments (2000 x 19456 fp32
+// outputs, K = 2560, 256 x 128 tiles: 251.7 -> 238.5 us).  (mw, nw): the wave's first output; acc as in
+// gemm_qknr_store.  The caller has passed a barrier since the k loop's last LDS read.
+template <typename TO, bool AF, int AM, int AN, bool SPLIT, bool SWIGLU>
+__device__ __forceinline__ void gemm_wave_store(const f32x16 (&acc)[AN][AM], char* wlds, int mw, int nw,
+                                                float* __restrict__ part, TO* C, int64_t ldc, const TO* cin,
+                                                int64_t ldcin, const TO* __restrict__ bias, int M, int N, float alpha,
+                                                float beta) {
+  using TS = std::conditional_t<SWIGLU, TO, float>;          // what is staged
+  constexpr int COLS = SWIGLU ? 16 * AN : 32 * AN;           // staged (output) columns of the wave
+  constexpr int ROW = COLS * (int)sizeof(TS) + 16;           // bytes per staged row
+  constexpr int E = SWIGLU ? 16 / (int)sizeof(TO) : 4;       // outputs per 16-byte chunk
+  constexpr int CH = COLS / E, STEPS = 32 * CH / 64;         // chunks per row, chunks per lane
+  const int lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
+  const int NO = SWIGLU ? N / 2 : N, n0 = SWIGLU ? nw / 2 : nw;
+  const bool vec = SPLIT || (((reinterpret_cast<uintptr_t>(C) | (cin ? reinterpret_cast<uintptr_t>(cin) : 0) |
+                               (bias ? reinterpret_cast<uintptr_t>(bias) : 0)) & 15) == 0 &&
+                             ((ldc | (cin ? ldcin : 0)) & 7) == 0);
 #pragma unroll
-    for (int b = 0; b < WTM; ++b) {
-      const int m = m0 + wm + 32 * b + r;
-      if (m >= M) continue;
-#pragma unroll
-      for (int a = 0; a < AN; ++a)
-#pragma unroll
-        for (int q = 0; q < 4; q += 2) {
-          const int f = (n0 + wn + 32 * a) / 2 + 4 * q + 4 * g;
-          if (f >= NH) continue;
-          float v[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            if constexpr (AF)
-              v[e] = silu_ref(acc[a][b][4 * q + e]) * acc[a][b][4 * q + 4 + e];
-            else
-              v[e] = silu_ref(round_bf16(acc[a][b][4 * q + e])) * round_bf16(acc[a][b][4 * q + 4 + e]);
-          }
-          store4<TO>(C, (int64_t)m * ldc + f, v, vec, 4);
-        }
-    }
-    return;
-  }
-#pragma unroll
-  for (int b = 0; b < WTM; ++b) {
-    const int m = m0 + wm + 32 * b + r;
-    if (m >= M) continue;
+  for (int b = 0; b < AM; ++b) {
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int a = 0; a < AN; ++a)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int n = n0 + wn + 32 * a + 8 * q + 4 * g;
-        if (n >= N) continue;
-        float v[4];
+      for (int q = 0; q < 4; q += SWIGLU ? 2 : 1) {
+        if constexpr (SWIGLU) {
+          float v[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          v[e] = (n + e < N) ? epilogue<TO>(acc[a][b][4 * q + e], alpha, beta, cin, ldcin, bias, m, n + e) : 0.f;
-        store4<TO>(C, (int64_t)m * ldc + n, v, vec, min(4, N - n));
+          for (int e = 0; e < 4; ++e)
+            v[e] = AF ? silu_ref(acc[a][b][4 * q + e]) * acc[a][b][4 * q + 4 + e]
+                      : silu_ref(round_bf16(acc[a][b][4 * q + e])) * round_bf16(acc[a][b][4 * q + 4 + e]);
+          TO* dst = reinterpret_cast<TO*>(wlds + r * ROW) + 16 * a + 4 * q + 4 * g;
+          if constexpr (sizeof(TO) == 2)
+            *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+          else
+            *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
+        } else {
+          *reinterpret_cast<float4*>(reinterpret_cast<float*>(wlds + r * ROW) + 32 * a + 8 * q + 4 * g) =
+              make_float4(acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]);
+        }
       }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int st = 0; st < STEPS; ++st) {
+      const int l = st * 64 + lane, row = l / CH, c = l % CH * E;
+      const int m = mw + 32 * b + row, n = n0 + c;
+      const uint4 x = *reinterpret_cast<const uint4*>(wlds + row * ROW + c * (int)sizeof(TS));
+      if (m >= M || n >= NO) continue;
+      if constexpr (SPLIT) {
+        *reinterpret_cast<uint4*>(part + (int64_t)m * N + n) = x;   // N % 4 == 0
+      } else if constexpr (SWIGLU) {
+        TO* dst = C + (int64_t)m * ldc + n;                         // N / 2 is a multiple of 8
+        if (vec) {
+          *reinterpret_cast<uint4*>(dst) = x;
+        } else {
+          const TO* xe = reinterpret_cast<const TO*>(&x);
+#pragma unroll
+          for (int e = 0; e < E; ++e) dst[e] = xe[e];
+        }
+      } else {
+        const float f[4] = {__uint_as_float(x.x), __uint_as_float(x.y), __uint_as_float(x.z), __uint_as_float(x.w)};
+        float v[4];
+        if (vec && n + 4 <= N) {
+          float ci[4] = {0.f, 0.f, 0.f, 0.f}, bi[4] = {0.f, 0.f, 0.f, 0.f};
+          auto ld4 = [](const TO* p, float (&o)[4]) {
+            if constexpr (sizeof(TO) == 2) {
+              const uint2 u = *reinterpret_cast<const uint2*>(p);
+              o[0] = lo_bf16(u.x); o[1] = hi_bf16(u.x); o[2] = lo_bf16(u.y); o[3] = hi_bf16(u.y);
+            } else {
+              const float4 u = *reinterpret_cast<const float4*>(p);
+              o[0] = u.x; o[1] = u.y; o[2] = u.z; o[3] = u.w;
+            }
+          };
+          const bool has_c = cin != nullptr && beta != 0.f;
+          if (has_c) ld4(cin + (int64_t)m * ldcin + n, ci);
+          if (bias != nullptr) ld4(bias + n, bi);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            v[e] = alpha * f[e];
+            if (has_c) v[e] += beta * ci[e];
+            if (bias != nullptr) v[e] += bi[e];
+          }
+          store4<TO>(C, (int64_t)m * ldc + n, v, true, 4);
+        } else {
+          const int valid = min(4, N - n);
+          for (int e = 0; e < valid; ++e)
+            Elem<TO>::store(C, (int64_t)m * ldc + n + e,
+                            epilogue<TO>(f[e], alpha, beta, cin, ldcin, bias, m, n + e));
+        }
+      }
+    }
+  }
+}
+
+// TA = float (fp32 activations, the reference's float32 arithmetic): A stays fp32 in LDS, and each value
+// a of a fragment is split into bf16 hi = bf16(a) and lo = bf16(a - hi) (a - hi is exact in fp32); every
+// 16-wide step then runs two MFMAs into the same accumulator, W * hi and W * lo.  The weights are exactly
+// bf16, so each product is W * a up to the 2^-17 relative error of hi + lo, fp32 accumulate; the
+// epilogues keep their fp32 values (no bf16 rounding of the SwiGLU operands or of the qk-norm + RoPE
+// input) and store fp32.
+//
+// What bounds it: for a few hundred rows, the latency of the loads and of the LDS and MFMA chain of each
+// k-step; for thousands of rows, the matrix cores and the power they draw.  So A and B rows go from
+// memory straight to LDS (buffer_load ... lds, 16 bytes a lane): a stage of the k loop costs no registers,
+// up to five of them are in flight, and there is one barrier per stage.  A wave's copy writes 1 KiB of
+// consecutive LDS bytes, so rows are stored without padding and the 16-byte chunks of a row are permuted
+// instead (chunk c of row i at place c ^ swz(i)): the 16 lanes that one cycle of a fragment read serves
+// then fall on 16 different bank groups (no bank conflicts counted).  Measured against the register-staged
+// kernel before it (two LDS buffers, 64 x 64 to 128 x 128 tiles), one call, weights from HBM:
+//   bf16  512 x 4096 x 1024  13.0 ->  9.4 us     fp32  512 x 4096 x 1024  19.3 -> 14.8 us
+//   bf16 1000 x 4096 x 1024  19.9 -> 14.4 us     fp32 1000 x 4096 x 1024  30.4 -> 23.1 us
+//   bf16 1000 x 6144 x 1024  30.9 -> 20.1 us     fp32 1000 x 6144 x 1024  55.1 -> 33.0 us
+//   bf16 2000 x 19456 x 2560  339 ->  240 us     fp32 2000 x 19456 x 2560  600 -> 405 us
+// Rows past M or N repeat the last one and are never stored; columns past the k range read as zero.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// 64 lanes x 16 bytes from rsrc at byte voff (per lane) + soff to LDS byte address lds + 16 lane.
+// Asynchronous: complete once a later s_waitcnt vmcnt says so.  (Inline asm rather than the builtin,
+// after which the compiler waits for every copy in flight before it reads any LDS.  m0 is reserved:
+// the compiler sets it anew before each use of its own.)
+__device__ __forceinline__ void copy_to_lds16(u32x4 rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :
+               : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
+               : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_vmem() {
+  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
+}
+// Wait until at most `left` stages of LPS copies each are in flight (left <= MAX).
+template <int LPS, int MAX>
+__device__ __forceinline__ void wait_stages(int left) {
+  if constexpr (MAX <= 0) {
+    wait_vmem<0>();
+  } else {
+    if (left >= MAX)
+      wait_vmem<LPS * MAX>();
+    else
+      wait_stages<LPS, MAX - 1>(left);
+  }
+}
+__device__ __forceinline__ u32x4 raw_rsrc(const void* base, uint32_t bytes) {
+  const uint64_t p = reinterpret_cast<uint64_t>(base);
+  u32x4 r;
+  r[0] = __builtin_amdgcn_readfirstlane((uint32_t)p);
+  r[1] = __builtin_amdgcn_readfirstlane((uint32_t)(p >> 32));
+  r[2] = __builtin_amdgcn_readfirstlane(bytes);
+  r[3] = 0x00020000u;
+  return r;
+}
+
+// A workgroup of WM x WN waves, each 32 AM x 32 AN outputs; NST stages of KS columns in LDS.
+template <typename TA, int AM, int AN, int WM, int WN, int KS>
+struct DmaTile {
+  static constexpr int GM = 32 * AM * WM, GN = 32 * AN * WN, NW = WM * WN;
+  static constexpr int CA = KS * (int)sizeof(TA) / 16, CB = KS * 2 / 16;   // 16-byte chunks per row
+  static constexpr int ABYTES = GM * CA * 16, BBYTES = GN * CB * 16, STAGE = ABYTES + BBYTES;
+  static constexpr int LA = GM * CA / (64 * NW), LB = GN * CB / (64 * NW); // copies per wave and stage
+  static_assert(GM * CA % (64 * NW) == 0 && GN * CB % (64 * NW) == 0, "whole copies");
+};
+// Rows that share one place of a chunk: 16 / C rows fill the 256 bytes of the 64 banks.
+template <int C>
+__device__ __forceinline__ int lds_swz(int row) {
+  static_assert(C == 4 || C == 8 || C == 16, "4, 8 or 16 chunks per row");
+  return (row / (16 / C)) & (C - 1);
+}
+
+template <typename TO, int AM, int AN, int WM, int WN, int KS, int NST, bool SPLIT, bool SWIGLU, bool QKNR,
+          typename TA>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(
+    const TA* __restrict__ A, int64_t lda, const uint16_t* __restrict__ B, int64_t ldb, TO* C, int64_t ldc,
+    const TO* cin, int64_t ldcin, const TO* __restrict__ bias, int M, int N, int K, float alpha, float beta,
+    int splits, int kchunk, float* __restrict__ part, QknrArgs qa) {
+  using T = DmaTile<TA, AM, AN, WM, WN, KS>;
+  constexpr bool AF = std::is_same<TA, float>::value;
+  constexpr int GM = T::GM, GN = T::GN, NW = T::NW, LPS = T::LA + T::LB;
+  constexpr int WLDS = 32 * (32 * AN * 4 + 16);  // a wave's 32 output rows, fp32 (gemm_wave_store)
+  constexpr int EPI = QKNR ? GM * (128 + 16 / (int)sizeof(TA)) * (int)sizeof(TA) : NW * WLDS;
+  constexpr int BYTES = NST * T::STAGE > EPI ? NST * T::STAGE : EPI;
+  __shared__ __attribute__((aligned(1024))) uint16_t smem[BYTES / 2];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int r = lane & 31, g = lane >> 5;
+  int bid = blockIdx.x;
+  if ((gridDim.x & 7) == 0) bid = (bid & 7) * (gridDim.x >> 3) + (bid >> 3);
+  const int tiles_m = (M + GM - 1) / GM;
+  const int tile = SPLIT ? bid / splits : bid, split = SPLIT ? bid % splits : 0;
+  const int m0 = tile % tiles_m * GM, n0 = tile / tiles_m * GN;
+  const int wm = wave / WN * 32 * AM, wn = wave % WN * 32 * AN;
+  const int kbeg = split * kchunk, klen = min(K, kbeg + kchunk) - kbeg, nk = (klen + KS - 1) / KS;
+
+  const int mrows = min(GM, M - m0), nrows = min(GN, N - n0);
+  const u32x4 ra = raw_rsrc(A + (int64_t)m0 * lda + kbeg, (uint32_t)(((int64_t)(mrows - 1) * lda + klen) * sizeof(TA)));
+  const u32x4 rb = raw_rsrc(B + (int64_t)n0 * ldb + kbeg, (uint32_t)(((int64_t)(nrows - 1) * ldb + klen) * 2));
+  // (128 rows of either operand fit 2 GiB, so the up to 256 of a tile fit 32-bit byte offsets.)
+  // Copy i of a stage holds chunk (i NW + wave) 64 + lane of its rows.  The copies of a wave are a
+  // multiple of 16 rows apart, so the lane's place in the row -- and its first column ka, kb -- is the
+  // same in each.
+  uint32_t va[T::LA], vb[T::LB];
+  const int l0 = wave * 64 + lane;
+  static_assert(NW * 64 / T::CA % 16 == 0 && NW * 64 / T::CB % 16 == 0, "copies whole swizzle periods apart");
+  const int ca = (l0 % T::CA) ^ lds_swz<T::CA>(l0 / T::CA), cb = (l0 % T::CB) ^ lds_swz<T::CB>(l0 / T::CB);
+  const int ka = ca * (16 / (int)sizeof(TA)), kb = cb * 8;
+#pragma unroll
+  for (int i = 0; i < T::LA; ++i)
+    va[i] = (uint32_t)min((i * NW * 64 + l0) / T::CA, mrows - 1) * (uint32_t)(lda * sizeof(TA)) + 16u * ca;
+#pragma unroll
+  for (int i = 0; i < T::LB; ++i)
+    vb[i] = (uint32_t)min((i * NW * 64 + l0) / T::CB, nrows - 1) * (uint32_t)(ldb * 2) + 16u * cb;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
+  // Copy i of this wave's LPS copies of stage t into buffer buf.  A chunk past the k range (K % 8 == 0:
+  // all in or all out) takes an offset past the buffer's, which reads zero.
+  auto issue_one = [&](int t, int buf, int i) {
+    const uint32_t base = lds0 + (uint32_t)(buf * T::STAGE + wave * 1024);
+    if (i < T::LA)
+      copy_to_lds16(ra, t * KS + ka < klen ? va[i < T::LA ? i : 0] : 0xffffffffu,
+                    (uint32_t)(t * KS * (int)sizeof(TA)), base + i * NW * 1024);
+    else
+      copy_to_lds16(rb, t * KS + kb < klen ? vb[i < T::LA ? 0 : i - T::LA] : 0xffffffffu, (uint32_t)(t * KS * 2),
+                    base + T::ABYTES + (i - T::LA) * NW * 1024);
+  };
+
+  f32x16 acc[AN][AM];
+#pragma unroll
+  for (int a = 0; a < AN; ++a)
+#pragma unroll
+    for (int b = 0; b < AM; ++b)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) acc[a][b][j] = 0.f;
+
+  // Fragments of one 16-wide k step: B rows, and A rows as stored (fp32: two 16-byte halves) until
+  // split_a makes them bf16 (fp32: hi and lo).
+  constexpr int AW = AF ? 2 : 1;
+  struct Frag {
+    uint4 b[AN], a[AM][AW];
+  };
+  auto read_frag = [&](Frag& f, int buf, int kc) {
+    const char* as = reinterpret_cast<const char*>(smem) + buf * T::STAGE;
+    const char* bs = as + T::ABYTES;
+#pragma unroll
+    for (int b = 0; b < AM; ++b) {
+      const int row = wm + 32 * b + r;
+#pragma unroll
+      for (int h = 0; h < AW; ++h)
+        f.a[b][h] = *reinterpret_cast<const uint4*>(as + row * (T::CA * 16) +
+                                                    (((AW * (2 * kc + g) + h) ^ lds_swz<T::CA>(row)) * 16));
+    }
+#pragma unroll
+    for (int a = 0; a < AN; ++a) {
+      const int row = wn + 32 * a + r;
+      f.b[a] = *reinterpret_cast<const uint4*>(bs + row * (T::CB * 16) + (((2 * kc + g) ^ lds_swz<T::CB>(row)) * 16));
+    }
+  };
+  auto split_a = [&](Frag& f) {
+    if constexpr (AF) {
+#pragma unroll
+      for (int b = 0; b < AM; ++b) {
+        const float4 x = __builtin_bit_cast(float4, f.a[b][0]), y = __builtin_bit_cast(float4, f.a[b][AW - 1]);
+        const uint32_t h0 = pack_bf16x2(x.x, x.y), h1 = pack_bf16x2(x.z, x.w), h2 = pack_bf16x2(y.x, y.y),
+                       h3 = pack_bf16x2(y.z, y.w);
+        f.a[b][0] = make_uint4(h0, h1, h2, h3);
+        f.a[b][AW - 1] = make_uint4(pack_bf16x2(x.x - lo_bf16(h0), x.y - hi_bf16(h0)),
+                                    pack_bf16x2(x.z - lo_bf16(h1), x.w - hi_bf16(h1)),
+                                    pack_bf16x2(y.x - lo_bf16(h2), y.y - hi_bf16(h2)),
+                                    pack_bf16x2(y.z - lo_bf16(h3), y.w - hi_bf16(h3)));
+      }
+    }
+  };
+  auto multiply = [&](const Frag& f, int pl, auto&& between) {
+#pragma unroll
+    for (int a = 0; a < AN; ++a) {
+#pragma unroll
+      for (int b = 0; b < AM; ++b)
+        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(f.b[a]), as_bf16x8(f.a[b][pl]), acc[a][b], 0, 0, 0);
+      between(a);
+    }
+  };
+  auto nothing = [](int) {};
+  // One 16-wide step: read the next step's fragments, multiply this one's; with fp32 activations the
+  // next fragments are split in the shadow of the second plane's products.
+  auto step = [&](Frag& cur, Frag& nxt, int buf, int kc, auto&& between) {
+    read_frag(nxt, buf, kc);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(cur, 0, between);
+    if constexpr (AF) {
+      __builtin_amdgcn_sched_barrier(0);
+      split_a(nxt);
+      multiply(cur, AW - 1, nothing);
+#pragma unroll
+      for (int i = 0; i < AN * AM; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                            // one MFMA
+        __builtin_amdgcn_sched_group_barrier(0x2, (24 + AN - 1) / AN, 0);           // its share of the split
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  // The fragments of the next 16-wide step are read before the current one is multiplied.  The last
+  // step of a stage is multiplied after the barrier that opens the next stage: there every wave's
+  // copies of that stage are complete, and every wave has read all of this stage, whose buffer takes
+  // the copies of the stage NST later.  Those are issued one by one between the products of the steps
+  // that follow, up to the next stage's barrier: issued together they keep the matrix cores waiting
+  // for the address unit (64 bytes per cycle).
+  constexpr int KC = KS / 16, ALL = KC * AN;
+  Frag fr[2];
+  if (nk > 0) {
+#pragma unroll
+    for (int s = 0; s < NST; ++s)
+      if (s < nk) {
+#pragma unroll
+        for (int i = 0; i < LPS; ++i) issue_one(s, s, i);
+      }
+    wait_stages<LPS, NST - 1>(nk - 1);
+    __builtin_amdgcn_s_barrier();
+    read_frag(fr[0], 0, 0);
+    split_a(fr[0]);
+    int buf = 0;
+    // Slots sl0 .. sl0 + AN - 1 of the ALL between two barriers: the copies of stage it.
+    auto copies = [&](int sl0, int it, int ibuf) {
+      return [&, sl0, it, ibuf](int i) {
+        const int k0 = (sl0 + i) * LPS / ALL, k1 = (sl0 + i + 1) * LPS / ALL;
+        if (k1 > k0) {
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int k = 0; k < LPS; ++k)
+            if (k >= k0 && k < k1) issue_one(it, ibuf, k);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+    };
+    constexpr int kLgkm0 = 0xc07f;  // s_waitcnt lgkmcnt(0)
+#pragma unroll
+    for (int kc = 0; kc + 1 < KC; ++kc) step(fr[kc & 1], fr[(kc + 1) & 1], 0, kc + 1, nothing);
+    int t = 0;
+    // Entering an iteration: stage t is read, its last step not yet multiplied, and stages up to
+    // t + NST - 1 are requested.
+    for (; t + NST < nk; ++t) {
+      __builtin_amdgcn_s_waitcnt(kLgkm0);
+      wait_vmem<LPS*(NST - 2)>();
+      const int ibuf = buf;
+      buf = buf == NST - 1 ? 0 : buf + 1;
+      __builtin_amdgcn_s_barrier();
+      step(fr[1], fr[0], buf, 0, copies(0, t + NST, ibuf));
+#pragma unroll
+      for (int kc = 0; kc + 1 < KC; ++kc)
+        step(fr[kc & 1], fr[(kc + 1) & 1], buf, kc + 1, copies((kc + 1) * AN, t + NST, ibuf));
+    }
+    for (; t + 1 < nk; ++t) {  // nothing left to request
+      __builtin_amdgcn_s_waitcnt(kLgkm0);
+      wait_stages<LPS, NST - 2>(nk - 2 - t);
+      buf = buf == NST - 1 ? 0 : buf + 1;
+      __builtin_amdgcn_s_barrier();
+      step(fr[1], fr[0], buf, 0, nothing);
+#pragma unroll
+      for (int kc = 0; kc + 1 < KC; ++kc) step(fr[kc & 1], fr[(kc + 1) & 1], buf, kc + 1, nothing);
+    }
+    multiply(fr[1], 0, nothing);
+    if constexpr (AF) multiply(fr[1], AW - 1, nothing);
+  }
+  __syncthreads();  // the tile is stored by way of the loop's LDS
+  if constexpr (QKNR) {
+    gemm_qknr_store<TA, AM, AN, GM, GN, NW>(acc, smem, m0, n0, wm, wn, M, N, qa);
+  } else {
+    gemm_wave_store<TO, AF, AM, AN, SPLIT, SWIGLU>(acc, reinterpret_cast<char*>(smem) + wave * WLDS, m0 + wm, n0 + wn,
+                                                   SPLIT ? part + (int64_t)split * M * N : nullptr, C, ldc, cin, ldcin,
+                                                   bias, M, N, alpha, beta);
   }
 }
 
@@ -712,23 +830,48 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const TA* __restrict_
     }
 }
 
-// Launch plan of the MFMA tile kernel for a bf16 [M, K] x [N, K]^T product.
+// The tiles, and what the choice among them rests on: microseconds of one 64-wide k-step with every CU
+// busy (from calls of 200 to 2000 rows; bf16 and fp32 activations) and of a tile's prologue and
+// epilogue.  Per output the large tiles cost the least, but a call takes as many rounds of 256
+// workgroups as its tiles need, so the choice is the smallest ceil(tiles / CUs) * (steps * step + ends).
+// For example 512 x 4096 x 1024 (fp32): 256 tiles of 64 x 128 14.8 us, 128 of 128 x 128 18.9, 512 of
+// 64 x 64 16.7; 1000 x 6144 x 1024: 192 of 128 x 256 33.0 us, 96 of 256 x 256 42, 384 of 128 x 128 40.
+struct TileCost {
+  int gm, gn;
+  float step, ends;
+};
+constexpr int kTiles = 5;
+constexpr TileCost kTileBf16[kTiles] = {
+    {64, 64, .20f, 1.f}, {64, 128, .38f, 1.5f}, {128, 128, .65f, 2.f}, {256, 128, .98f, 3.f}, {256, 256, 1.7f, 5.f}};
+constexpr TileCost kTileF32[kTiles] = {
+    {64, 64, .50f, 1.f}, {64, 128, .71f, 1.5f}, {128, 128, 1.19f, 2.f}, {128, 256, 1.75f, 3.f}, {256, 256, 3.2f, 5.f}};
+constexpr int kCUs = 256;
+
+inline float tile_cost(const TileCost& t, int64_t M, int64_t N, int64_t K, int splits) {
+  const int64_t blocks = ((M + t.gm - 1) / t.gm) * ((N + t.gn - 1) / t.gn) * splits;
+  const float steps = (float)((K + 63) / 64) / (float)splits;
+  return (float)((blocks + kCUs - 1) / kCUs) * (steps * t.step + t.ends);
+}
+// The tile (from `first` on) of a product split `splits` ways; its cost in *cost if given.
+inline int choose_tile(bool f32, int M, int N, int K, int splits, int first = 0, float* cost = nullptr) {
+  int best = first;
+  float low = 0.f;
+  for (int i = first; i < kTiles; ++i) {
+    const float c = tile_cost(f32 ? kTileF32[i] : kTileBf16[i], M, N, K, splits);
+    if (i == first || c < low) {
+      low = c;
+      best = i;
+    }
+  }
+  if (cost) *cost = low;
+  return best;
+}
+
+// Launch plan of the MFMA tile kernel for a bf16 (or fp32) [M, K] x bf16 [N, K]^T product.
 struct GemmPlan {
   bool mfma = false;  // the MFMA tile kernel applies (else the skinny or generic kernel)
-  int wtm = 1, wtn = 1, tiles_m = 0, tiles_n = 0, splits = 1, kchunk = 0;
-  int64_t tiles = 0;
+  int tile = 0, splits = 1, kchunk = 0;
 };
-
-// Tile (64 wtm) x (64 wtn) of a product that does not split K.
-inline void plain_tile(int M, int N, int& wtm, int& wtn) {
-  const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
-  if (t128 >= kGemmT128Min) {
-    wtm = wtn = 2;
-  } else {
-    wtm = kGemmSmallWTM;
-    wtn = kGemmSmallWTN;
-  }
-}
 
 // aligned: both operands start on 16 bytes.  bf16: bf16 weights B with bf16 (a_bytes 2) or fp32
 // (a_bytes 4, split into hi + lo) activations A.
@@ -736,92 +879,84 @@ GemmPlan gemm_plan(bool aligned, int64_t lda, int64_t ldb, int M, int N, int K, 
                    int a_bytes = 2) {
   GemmPlan p;
   const int64_t lim = int64_t(1) << 31;
-  if (!(bf16 && trans_b && M > SK_MAXM && K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned &&
-        (int64_t)g_tile(2) * lda * a_bytes < lim && (int64_t)g_tile(2) * ldb * 2 < lim))
+  if (!(bf16 && trans_b && M > SK_MAXM && K > 0 && K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned &&
+        128 * lda * a_bytes < lim && 128 * ldb * 2 < lim))
     return p;
   p.mfma = true;
-  // The K split is decided on the 64-tile count, whatever tile then runs it, so a shape's k ranges
-  // -- and with them its sums, bit for bit -- do not depend on the tile: split when 64-tiles would
-  // leave CUs idle and K is long, over up to 8 workgroups per tile.
-  const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
-  const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
   p.kchunk = K;
-  if (t64 < 256 && K >= 1024 && N % 4 == 0) {
-    const int64_t want = kGemmSplitTarget / t64;
-    const int splits = want < 1 ? 1 : (want > kMaxSplits ? kMaxSplits : (int)want);
-    if (splits > 1) {
-      p.kchunk = ((K + splits - 1) / splits + 127) / 128 * 128;   // whole k-steps of 64 and 128
-      p.splits = (K + p.kchunk - 1) / p.kchunk;
+  // The K split (the same for bf16 and fp32 activations, so that kh_gemm_split_count needs no type) is
+  // the cheapest for fp32 ones: a split adds the partials' way through memory (0.35 us a MB) and about
+  // 1 us, and pays where the tiles of whole sums leave CUs idle.  1000 x 1024 x 3072 fp32: 64 x 64 tiles
+  // unsplit 26.8 us, 64 x 128 split in two 19.9; 512 x 1024 x 3072: 23.7 us unsplit, 13.3 split in four.
+  if (K >= 512 && N % 4 == 0) {
+    float low = 0.f;
+    for (int sp = 1; sp <= kMaxSplits; ++sp) {
+      const int kchunk = ((K + sp - 1) / sp + 127) / 128 * 128;
+      if (sp > 1 && (K + kchunk - 1) / kchunk != sp) continue;
+      float c;
+      choose_tile(true, M, N, K, sp, 0, &c);
+      if (sp > 1) c += 1.f + 0.35e-6f * 4.f * (float)sp * (float)M * (float)N;
+      if (sp == 1 || c < low) {
+        low = c;
+        p.splits = sp;
+        p.kchunk = sp > 1 ? kchunk : K;
+      }
     }
   }
-  // 128-tiles when they fill the chip (256 CUs), else smaller tiles for more workgroups.
-  if (p.splits > 1) {
-    p.wtm = a_bytes == 4 ? kGemmSplitF32WTM : kGemmSplitWTM;
-    p.wtn = a_bytes == 4 ? kGemmSplitF32WTN : kGemmSplitWTN;
-  } else {
-    plain_tile(M, N, p.wtm, p.wtn);
-  }
-  (void)t128;
-  p.tiles_m = (M + g_tile(p.wtm) - 1) / g_tile(p.wtm);
-  p.tiles_n = (N + g_tile(p.wtn) - 1) / g_tile(p.wtn);
-  p.tiles = (int64_t)p.tiles_m * p.tiles_n;
+  p.tile = choose_tile(a_bytes == 4, M, N, K, p.splits);
   return p;
 }
 
-// One launch of the tile kernel with tile (64 WTM) x (64 WTN) and k-step KS.
-template <typename TO, int WTM, int WTN, int KS, bool SWIGLU = false, typename TA = uint16_t>
-void go_tiles(int nblk, int splits, const TA* A, int64_t lda, const uint16_t* B, int64_t ldb, TO* C,
-              int64_t ldc, const TO* CI, int64_t ldcin, const TO* BI, int M, int N, int K, float alpha, float beta,
-              int tiles_n, int kchunk, float* part) {
-  // fp32 activations hold twice the A chunks per stage: two stages in flight keep the ring in registers
-  constexpr int PF = std::is_same<TA, float>::value ? 2 : kGemmPrefetch;
-  constexpr int NW = gemm_waves<WTM, WTN>();
-  if (!SWIGLU && splits > 1)
-    gemm_bf16_nt_kernel<TO, WTM, WTN, KS, true, kGemmSplitPrefetch, false, false, TA, NW><<<nblk, NW * 64, 0,
-                                                                                            stream()>>>(
-        A, lda, B, ldb, C, ldc, CI, ldcin, BI, M, N, K, alpha, beta, tiles_n, splits, kchunk, part, QknrArgs{});
-  else
-    gemm_bf16_nt_kernel<TO, WTM, WTN, KS, false, PF, SWIGLU, false, TA, NW><<<nblk, NW * 64, 0, stream()>>>(
-        A, lda, B, ldb, C, ldc, CI, ldcin, BI, M, N, K, alpha, beta, tiles_n, 1, K, nullptr, QknrArgs{});
+enum TileUse { USE_PLAIN, USE_SPLIT, USE_SWIGLU, USE_QKNR };
+
+// One launch of the tile kernel: AM x AN blocks of 32 x 32 outputs per wave, WM x WN waves, NST stages
+// of KS columns in LDS.
+template <typename TO, typename TA, TileUse USE, int AM, int AN, int WM, int WN, int KS, int NST>
+int go_tile(const TA* A, int64_t lda, const uint16_t* B, int64_t ldb, TO* C, int64_t ldc, const TO* CI, int64_t ldcin,
+            const TO* BI, int M, int N, int K, float alpha, float beta, int splits, int kchunk, float* part,
+            const QknrArgs& qa) {
+  using T = DmaTile<TA, AM, AN, WM, WN, KS>;
+  const int64_t blocks = (int64_t)((M + T::GM - 1) / T::GM) * ((N + T::GN - 1) / T::GN) * splits;
+  KH_REQUIRE(blocks <= INT32_MAX, "kh_gemm: grid too large");
+  gemm_tile_kernel<TO, AM, AN, WM, WN, KS, NST, USE == USE_SPLIT, USE == USE_SWIGLU, USE == USE_QKNR, TA>
+      <<<(int)blocks, 64 * WM * WN, 0, stream()>>>(A, lda, B, ldb, C, ldc, CI, ldcin, BI, M, N, K, alpha, beta, splits,
+                                                   kchunk, part, qa);
+  KH_CHECK_LAUNCH();
+  return KH_OK;
 }
 
-// Dispatch on the plan's tile: 128 x 128 with k-step 64; 64 x 64 with k-step 128 when split or
-// with at most one tile per CU, else k-step 64 (C5 prefill qkv, 512 tiles: 11.75 -> 10.9 us with
-// k-step 64; gate/up, 768 tiles: 14.0 -> 16.1 us with k-step 128); 128 x 64 and 64 x 128 with
-// kGemmRectKS.  fp32 activations (TA float: two LDS planes of A) keep a k-step of 64 on 64 x 64
-// tiles, so that two workgroups still fit a CU's LDS.
-template <typename TO, bool SWIGLU = false, typename TA = uint16_t>
-void launch_tile_shape(int wtm, int wtn, int64_t tiles, int splits, const TA* A, int64_t lda,
-                       const uint16_t* B, int64_t ldb, TO* C, int64_t ldc, const TO* CI, int64_t ldcin, const TO* BI,
-                       int M, int N, int K, float alpha, float beta, int tiles_n, int kchunk, float* part) {
+// The tile kernel with tile `tile` of kTileBf16 / kTileF32.  k-steps of 64 columns; of 32 where two or
+// three stages of 64 do not fit the CU's 160 KiB of LDS.  64 x 128 fp32 tiles run four waves of 32 x 64
+// (each A fragment split by two waves, not four: 16.6 -> 14.8 us at 512 x 4096 x 1024).
+template <typename TO, typename TA, TileUse USE>
+int launch_tile(int tile, const TA* A, int64_t lda, const uint16_t* B, int64_t ldb, TO* C, int64_t ldc, const TO* CI,
+                int64_t ldcin, const TO* BI, int M, int N, int K, float alpha, float beta, int splits, int kchunk,
+                float* part, const QknrArgs& qa = QknrArgs{}) {
   constexpr bool AF = std::is_same<TA, float>::value;
-  const int nblk = (int)(tiles * splits);
-  if (wtm == 2 && wtn == 2)
-    go_tiles<TO, 2, 2, 64, SWIGLU, TA>(nblk, splits, A, lda, B, ldb, C, ldc, CI, ldcin, BI, M, N, K, alpha, beta,
-                                       tiles_n, kchunk, part);
-  else if (wtm == 2)
-    go_tiles<TO, 2, 1, kGemmRectKS, SWIGLU, TA>(nblk, splits, A, lda, B, ldb, C, ldc, CI, ldcin, BI, M, N, K, alpha,
-                                                beta, tiles_n, kchunk, part);
-  else if (wtn == 2)
-    go_tiles<TO, 1, 2, kGemmRectKS, SWIGLU, TA>(nblk, splits, A, lda, B, ldb, C, ldc, CI, ldcin, BI, M, N, K, alpha,
-                                                beta, tiles_n, kchunk, part);
-  else if (!AF && (splits > 1 || tiles <= 256))
-    go_tiles<TO, 1, 1, AF ? 64 : 128, SWIGLU, TA>(nblk, splits, A, lda, B, ldb, C, ldc, CI, ldcin, BI, M, N, K, alpha,
-                                                  beta, tiles_n, kchunk, part);
-  else
-    go_tiles<TO, 1, 1, 64, SWIGLU, TA>(nblk, splits, A, lda, B, ldb, C, ldc, CI, ldcin, BI, M, N, K, alpha, beta,
-                                       tiles_n, kchunk, part);
-}
-
-// The MFMA tile kernel for plan p: C (or, with part != nullptr and p.splits > 1, only the fp32
-// partials part[split][m][n]).
-template <typename TO, typename TA = uint16_t>
-void launch_gemm_tiles(const GemmPlan& p, const TA* A, int64_t lda, const uint16_t* B, int64_t ldb, TO* C,
-                       int64_t ldc, const TO* CI, int64_t ldcin, const TO* BI, int M, int N, int K, float alpha,
-                       float beta, float* part) {
-  const int splits = part ? p.splits : 1;
-  launch_tile_shape<TO, false, TA>(p.wtm, p.wtn, p.tiles, splits, A, lda, B, ldb, C, ldc, CI, ldcin, BI, M, N, K,
-                                   alpha, beta, p.tiles_n, p.kchunk, part);
+  auto go = [&](auto am, auto an, auto wm, auto wn, auto ks, auto nst) {
+    return go_tile<TO, TA, USE, decltype(am)::value, decltype(an)::value, decltype(wm)::value, decltype(wn)::value,
+                   decltype(ks)::value, decltype(nst)::value>(A, lda, B, ldb, C, ldc, CI, ldcin, BI, M, N, K, alpha,
+                                                              beta, splits, kchunk, part, qa);
+  };
+  auto c = [](auto v) { return v; };
+#define KH_I(v) c(std::integral_constant<int, (v)>{})
+  if constexpr (USE != USE_QKNR)
+    if (tile == 0) return go(KH_I(1), KH_I(1), KH_I(2), KH_I(2), KH_I(64), KH_I(AF ? 3 : 4));
+  if (tile <= 1) {
+    if constexpr (AF)
+      return go(KH_I(1), KH_I(2), KH_I(2), KH_I(2), KH_I(64), KH_I(4));
+    else
+      return go(KH_I(1), KH_I(1), KH_I(2), KH_I(4), KH_I(64), KH_I(6));
+  }
+  if (tile == 2) return go(KH_I(1), KH_I(2), KH_I(4), KH_I(2), KH_I(64), KH_I(AF ? 3 : 4));
+  if (tile == 3) {
+    if constexpr (AF)
+      return go(KH_I(1), KH_I(4), KH_I(4), KH_I(2), KH_I(32), KH_I(4));
+    else
+      return go(KH_I(2), KH_I(2), KH_I(4), KH_I(2), KH_I(64), KH_I(3));
+  }
+  return go(KH_I(2), KH_I(4), KH_I(4), KH_I(2), KH_I(32), KH_I(AF ? 3 : 4));
+#undef KH_I
 }
 
 // A has element type TA, B has T (bf16 weights may meet fp32 activations: TA float, T uint16_t).
@@ -837,17 +972,22 @@ int launch_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
   const GemmPlan p = gemm_plan(aligned16(a) && aligned16(b), lda, ldb, M, N, K, w_bf16, trans_b, (int)sizeof(TA));
   if constexpr (w_bf16) {
     if (p.mfma) {
-      KH_REQUIRE(p.tiles <= INT32_MAX / 8, "kh_gemm: grid too large");
-      float* part = nullptr;
-      if (p.splits > 1) part = (float*)scratch_alloc((size_t)p.splits * M * N * sizeof(float));
-      launch_gemm_tiles<TO, TA>(p, A, lda, (const uint16_t*)B, ldb, C, ldc, CI, ldcin, BI, M, N, K, alpha, beta, part);
-      if (part) {
-        gemm_splitk_reduce_kernel<TO><<<(int)(((int64_t)M * N / 4 + 255) / 256), 256, 0, stream()>>>(
-            part, p.splits, C, ldc, CI, ldcin, BI, M, N, alpha, beta);
-        scratch_free(part);  // stream-ordered reuse only
+      if (p.splits > 1) {
+        float* part = (float*)scratch_alloc((size_t)p.splits * M * N * sizeof(float));
+        if (part != nullptr) {
+          const int rc = launch_tile<float, TA, USE_SPLIT>(p.tile, A, lda, (const uint16_t*)B, ldb, nullptr, 0, nullptr,
+                                                           0, nullptr, M, N, K, alpha, beta, p.splits, p.kchunk, part);
+          if (rc == KH_OK)
+            gemm_splitk_reduce_kernel<TO><<<(int)(((int64_t)M * N / 4 + 255) / 256), 256, 0, stream()>>>(
+                part, p.splits, C, ldc, CI, ldcin, BI, M, N, alpha, beta);
+          scratch_free(part);  // stream-ordered reuse only
+          if (rc != KH_OK) return rc;
+          KH_CHECK_LAUNCH();
+          return KH_OK;
+        }
       }
-      KH_CHECK_LAUNCH();
-      return KH_OK;
+      return launch_tile<TO, TA, USE_PLAIN>(choose_tile(sizeof(TA) == 4, M, N, K, 1), A, lda, (const uint16_t*)B, ldb, C,
+                                            ldc, CI, ldcin, BI, M, N, K, alpha, beta, 1, K, nullptr);
     }
     if (trans_b && M == 1) {
       constexpr bool EX = std::is_same<TA, float>::value;
@@ -876,41 +1016,21 @@ int launch_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
   return KH_OK;
 }
 
-// The fused SwiGLU projection: the MFMA tile kernel with the SWIGLU epilogue, tiles chosen as in
-// launch_gemm, never split over K (the epilogue needs whole sums).  TA = TO: bf16, or fp32
-// activations in and out.
+// The fused SwiGLU projection: the MFMA tile kernel with the SWIGLU epilogue, never split over K (the
+// epilogue needs whole sums).  TA = TO: bf16, or fp32 activations in and out.
 template <typename TA>
 int launch_gemm_swiglu(const TA* X, int64_t ldx, const uint16_t* W, int64_t ldw, TA* H, int64_t ldh, int M, int N,
                        int K) {
-  int wtm = 1, wtn = 1;
-  // fp32 activations (two MFMAs per k-step) take 64 x 128 tiles: C5 gate/up 27.0-27.3 -> 23.7-23.8 us
-  // (128 x 64: 36.2 us); bf16 keeps the plain choice.  The tile never changes a sum.
-  if constexpr (std::is_same<TA, float>::value)
-    wtn = 2;
-  else
-    plain_tile(M, N, wtm, wtn);
-  const int tiles_m = (M + g_tile(wtm) - 1) / g_tile(wtm), tiles_n = (N + g_tile(wtn) - 1) / g_tile(wtn);
-  const int64_t tiles = (int64_t)tiles_m * tiles_n;
-  KH_REQUIRE(tiles <= INT32_MAX, "kh_gemm_swiglu: grid too large");
-  launch_tile_shape<TA, true, TA>(wtm, wtn, tiles, 1, X, ldx, W, ldw, H, ldh, nullptr, 0, nullptr, M, N, K, 1.f, 0.f,
-                                  tiles_n, K, nullptr);
-  KH_CHECK_LAUNCH();
-  return KH_OK;
+  return launch_tile<TA, TA, USE_SWIGLU>(choose_tile(sizeof(TA) == 4, M, N, K, 1), X, ldx, W, ldw, H, ldh, nullptr, 0,
+                                         nullptr, M, N, K, 1.f, 0.f, 1, K, nullptr);
 }
 
-// The fused QKV projection: 64 x 128 tiles (one head row of 128 per tile column), never split.
+// The fused QKV projection: tiles of whole head rows of 128, never split.
 template <typename TA>
 int launch_gemm_qk_norm_rope(const TA* X, int64_t ldx, const uint16_t* W, int64_t ldw, int M, int N, int K,
                              const QknrArgs& qa) {
-  const int tiles_m = (M + 63) / 64, tiles_n = N / 128;
-  const int64_t tiles = (int64_t)tiles_m * tiles_n;
-  KH_REQUIRE(tiles <= INT32_MAX, "kh_gemm_qk_norm_rope: grid too large");
-  constexpr int PF = std::is_same<TA, float>::value ? 2 : kGemmPrefetch;
-  constexpr int NW = gemm_waves<1, 2>();
-  gemm_bf16_nt_kernel<TA, 1, 2, kGemmRectKS, false, PF, false, true, TA, NW><<<(int)tiles, NW * 64, 0, stream()>>>(
-      X, ldx, W, ldw, nullptr, 0, nullptr, 0, nullptr, M, N, K, 1.f, 0.f, tiles_n, 1, K, nullptr, qa);
-  KH_CHECK_LAUNCH();
-  return KH_OK;
+  return launch_tile<TA, TA, USE_QKNR>(choose_tile(sizeof(TA) == 4, M, N, K, 1, 1), X, ldx, W, ldw, (TA*)nullptr, 0,
+                                       nullptr, 0, nullptr, M, N, K, 1.f, 0.f, 1, K, nullptr, qa);
 }
 
 }  // namespace
@@ -991,15 +1111,13 @@ int kh_gemm_splitk_partials(const void* a, int64_t lda, const void* b, int64_t l
   KH_REQUIRE(p.mfma && p.splits > 1 && p.splits == splits,
              "kh_gemm_splitk_partials: this product is not split %d ways (kh_gemm_split_count gives the count; "
              "operands must be 16-byte aligned with k and the leading dimensions multiples of 8)", splits);
-  KH_REQUIRE(p.tiles <= INT32_MAX / 8, "kh_gemm_splitk_partials: grid too large");
   if (a_dtype == KH_F32)
-    launch_gemm_tiles<float, float>(p, (const float*)a, lda, (const uint16_t*)b, ldb, nullptr, n, nullptr, 0, nullptr,
-                                    (int)m, (int)n, (int)k, 1.f, 0.f, part);
-  else
-    launch_gemm_tiles<float>(p, (const uint16_t*)a, lda, (const uint16_t*)b, ldb, nullptr, n, nullptr, 0, nullptr,
-                             (int)m, (int)n, (int)k, 1.f, 0.f, part);
-  KH_CHECK_LAUNCH();
-  return KH_OK;
+    return launch_tile<float, float, USE_SPLIT>(p.tile, (const float*)a, lda, (const uint16_t*)b, ldb, nullptr, 0,
+                                                nullptr, 0, nullptr, (int)m, (int)n, (int)k, 1.f, 0.f, p.splits, p.kchunk,
+                                                part);
+  return launch_tile<float, uint16_t, USE_SPLIT>(p.tile, (const uint16_t*)a, lda, (const uint16_t*)b, ldb, nullptr, 0,
+                                                 nullptr, 0, nullptr, (int)m, (int)n, (int)k, 1.f, 0.f, p.splits,
+                                                 p.kchunk, part);
 }
 
 int kh_gemm_swiglu(const void* x, int64_t ldx, const void* w_gu, int64_t ldw, void* h, int64_t ldh, int64_t m,
@@ -1016,7 +1134,7 @@ int kh_gemm_swiglu(const void* x, int64_t ldx, const void* w_gu, int64_t ldw, vo
   KH_REQUIRE(aligned16(x) && aligned16(w_gu), "kh_gemm_swiglu: x and w_gu must be 16-byte aligned");
   const int64_t lim = int64_t(1) << 31;
   const int xb = x_dtype == KH_F32 ? 4 : 2;
-  KH_REQUIRE((int64_t)g_tile(2) * ldx * xb < lim && (int64_t)g_tile(2) * ldw * 2 < lim,
+  KH_REQUIRE(128 * ldx * xb < lim && 128 * ldw * 2 < lim,
              "kh_gemm_swiglu: row stride too large");
   if (x_dtype == KH_F32)
     return launch_gemm_swiglu<float>((const float*)x, ldx, (const uint16_t*)w_gu, ldw, (float*)h, ldh, (int)m,
@@ -1084,7 +1202,7 @@ int kh_gemm_qk_norm_rope_table(const void* x, int64_t ldx, const void* w_qkv, in
   for (const void* p : al) KH_REQUIRE(aligned16(p), "kh_gemm_qk_norm_rope: operands must be 16-byte aligned");
   const int64_t lim = int64_t(1) << 31;
   const int xb = dtype == KH_F32 ? 4 : 2;
-  KH_REQUIRE((int64_t)g_tile(2) * ldx * xb < lim && (int64_t)g_tile(2) * ldw * 2 < lim,
+  KH_REQUIRE(128 * ldx * xb < lim && 128 * ldw * 2 < lim,
              "kh_gemm_qk_norm_rope: row stride too large");
   QknrArgs qa;
   const int64_t vec = 16 / xb;
