@@ -120,9 +120,17 @@ def check(rc: int, what: str = "") -> None:
         raise KandleHipError(f"{what or 'kandle_hip'} failed (code {rc}): {msg}")
 
 
+_functions: dict = {}  # name -> the library's entry point, bound on first use
+
+
 def call(name: str, *args) -> None:
     """Call an entry point and raise on a non-zero return code."""
-    check(getattr(load(), name)(*args), name)
+    fn = _functions.get(name)
+    if fn is None:
+        fn = _functions[name] = getattr(load(), name)
+    rc = fn(*args)
+    if rc != 0:
+        check(rc, name)
 
 
 def is_capturing() -> bool:
@@ -130,9 +138,13 @@ def is_capturing() -> bool:
     return bool(load().kh_is_capturing())
 
 
+_I64_ARRAYS = [C.c_int64 * max(1, n) for n in range(17)]
+
+
 def i64_array(values) -> C.Array:
     vals = [int(v) for v in values]
-    return (C.c_int64 * max(1, len(vals)))(*vals)
+    n = len(vals)
+    return (_I64_ARRAYS[n] if n < len(_I64_ARRAYS) else C.c_int64 * n)(*vals)
 
 
 def device_count() -> int:

@@ -113,7 +113,7 @@ def dispatch_matmul(a: Tensor, b: Tensor, c: Optional[Tensor] = None, alpha: flo
     M, K = a2[-2], a2[-1]
     if K != Kb:
         raise ValueError(f"matmul: inner dimensions differ ({K} vs {Kb}) for {tuple(ash)} @ {tuple(bsh)}")
-    batch_shape = list(np.broadcast_shapes(tuple(a2[:-2]), tuple(b2[:-2])))
+    batch_shape = list(np.broadcast_shapes(tuple(a2[:-2]), tuple(b2[:-2]))) if len(a2) > 2 or len(b2) > 2 else []
     out_shape = batch_shape + [M, N]
     if len(ash) == 1:
         out_shape.pop(-2)
@@ -127,7 +127,7 @@ def dispatch_matmul(a: Tensor, b: Tensor, c: Optional[Tensor] = None, alpha: flo
         output = _new(a, out_shape, out_dtype)
     variant = "mm" if not batch_shape else "bmm"
     cfg = MatmulDispatchResult(variant=variant, output=output, M=M, K=K, N=N, batch_shape=tuple(batch_shape),
-                               batch_size=int(np.prod(batch_shape)) if batch_shape else 1, transpose_a=False,
+                               batch_size=math.prod(batch_shape), transpose_a=False,
                                transpose_b=bool(transpose_b), alpha=float(alpha), beta=float(beta),
                                input_c=c.handle if c is not None else None,
                                bias=bias.handle if bias is not None else None)

@@ -21,6 +21,7 @@ from __future__ import annotations
 
 import ctypes as C
 import dataclasses
+import math
 from dataclasses import dataclass, field
 from typing import Optional, Sequence
 
@@ -311,10 +312,10 @@ def matmul(config: MatmulDispatchResult, a: HipTensorHandle, b: HipTensorHandle)
             tmp.append(Bm)
         if not out.is_contiguous():
             raise ValueError("matmul: output must be contiguous")
-        batch = int(np.prod(config.batch_shape)) if len(config.batch_shape) else 1
+        batch = math.prod(config.batch_shape)
         a_rows = A.numel // K if K else 0
         # Fold batch into M when A is a contiguous stack and B is shared (x W^T of a 3-D activation).
-        b_batched = len(Bm.shape) > 2 and int(np.prod(Bm.shape[:-2])) > 1
+        b_batched = len(Bm.shape) > 2 and math.prod(Bm.shape[:-2]) > 1
         if not b_batched and A.is_contiguous():
             _gemm_call(A, K, Bm, out, N, config, rows=a_rows, a_off=0, b_off=0, c_off=0)
             return
@@ -395,7 +396,7 @@ def rms_norm(inputs, params) -> HipTensorHandle:
     w = params.get("weight")
     if params.get("bias") is not None:
         raise ValueError("rms_norm: bias is not part of RMSNorm")
-    n = int(np.prod(ns))
+    n = math.prod(ns)
     xs = x if x.is_contiguous() else _materialize(x)
     try:
         rows = xs.numel // n if n else 0
@@ -542,7 +543,7 @@ class TensorIterator:
         self.num_outputs = len(outputs)
         self.num_inputs = len(self.operands) - self.num_outputs
         self.input_shape, self.output_shape = _shapes
-        self.output_numel = int(np.prod(self.output_shape)) if self.output_shape else 1
+        self.output_numel = math.prod(self.output_shape)
         axes, keep = _reduction if _reduction is not None else ((), False)
         self.reduction_axes = tuple(axes)
         self.is_reduction = bool(axes)
@@ -572,7 +573,8 @@ class TensorIterator:
         """Elementwise: the inputs broadcast to one shape; the output (allocated, in out_dtype or the
         promoted input dtype, when not given) has that shape."""
         if output is None:
-            shape = tuple(np.broadcast_shapes(*[tuple(h.shape) for h in inputs])) if inputs else ()
+            shape = tuple(np.broadcast_shapes(*[tuple(h.shape) for h in inputs])) if len(inputs) > 1 else \
+                tuple(inputs[0].shape) if inputs else ()
             output = HipTensorHandle.create_new(shape, out_dtype or _promote([h.dtype for h in inputs]))
         else:
             np.broadcast_shapes(tuple(output.shape), *[tuple(h.shape) for h in inputs])
@@ -608,7 +610,7 @@ class TensorIterator:
         out_shape = tuple(1 if i in red else x.shape[i] for i in range(nd)) if keep_dims else \
             tuple(x.shape[i] for i in kept)
         out = output if output is not None else HipTensorHandle.create_new(out_shape, out_dtype or x.dtype)
-        if out.numel != (int(np.prod(out_shape)) if out_shape else 1):
+        if out.numel != math.prod(out_shape):
             raise ValueError(f"reduction: output {tuple(out.shape)} for a result of {out_shape}")
         ops = [IteratorOperand(out, out.dtype, tuple(out.shape), tuple(out.strides), out.offset, True),
                IteratorOperand(x, x.dtype, tuple(x.shape), tuple(x.strides[i] for i in kept), x.offset, False,
@@ -761,8 +763,8 @@ def index_select(self_: HipTensorHandle, index: HipTensorHandle, params: dict, o
     t = self_ if self_.is_contiguous() else _materialize(self_)
     try:
         shape = list(t.shape) if nd else [1]
-        outer = int(np.prod(shape[:dim])) if dim else 1
-        inner = int(np.prod(shape[dim + 1:])) if dim + 1 < len(shape) else 1
+        outer = math.prod(shape[:dim])
+        inner = math.prod(shape[dim + 1:])
         if output.numel != outer * index.numel * inner:
             raise ValueError("index_select: output must hold len(index) entries along dim")
         _lib.call(
@@ -791,8 +793,8 @@ def argmax(it: TensorIterator) -> None:
         raise ValueError(f"argmax: axis out of range for a {nd}-d tensor")
     kept = [i for i in range(nd) if i not in axes]
     perm = kept + axes
-    R = int(np.prod([x.shape[a] for a in axes])) if axes else 1
-    P = int(np.prod([x.shape[i] for i in kept])) if kept else 1
+    R = math.prod([x.shape[a] for a in axes])
+    P = math.prod([x.shape[i] for i in kept])
     if R == 0:
         raise ValueError("argmax: reduction over an empty axis")
     out = it.output(0)
@@ -845,7 +847,7 @@ def linear_swiglu(x, w_gu, output) -> None:
         raise ValueError(f"linear_swiglu: x [..., {H}] and output [..., {I}] expected for w_gu {tuple(w_gu.shape)}")
     if x.strides[-1] != 1 or w_gu.strides[1] != 1 or output.strides[-1] != 1:
         raise ValueError("linear_swiglu: rows must be contiguous")
-    m = int(np.prod(x.shape[:-1])) if len(x.shape) > 1 else 1
+    m = math.prod(x.shape[:-1])
     if len(x.shape) > 2 and not (x.is_contiguous() and output.is_contiguous()):
         raise ValueError("linear_swiglu: batched operands must be contiguous")
     ldx = x.strides[-2] if len(x.shape) >= 2 else H

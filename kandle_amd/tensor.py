@@ -15,6 +15,7 @@ from __future__ import annotations
 
 import ctypes as C
 import itertools
+import math
 from typing import Optional, Sequence
 
 import numpy as np
@@ -27,17 +28,17 @@ _ids = itertools.count(1)
 
 def contiguous_strides(shape: Sequence[int]) -> list:
     strides, acc = [], 1
-    for s in reversed(list(shape)):
+    for s in reversed(shape):
         strides.append(acc)
-        acc *= max(int(s), 1)
-    return list(reversed(strides))
+        s = int(s)
+        if s > 1:
+            acc *= s
+    strides.reverse()
+    return strides
 
 
 def numel_of(shape: Sequence[int]) -> int:
-    n = 1
-    for s in shape:
-        n *= int(s)
-    return n
+    return math.prod([int(s) for s in shape])
 
 
 class HipStorage:
@@ -113,9 +114,9 @@ class HipTensorHandle:
 
     def __init__(self, storage: HipStorage, shape, dtype: str, strides=None, offset: int = 0):
         self.storage = storage
-        self.shape = tuple(int(s) for s in shape)
+        self.shape = tuple([int(s) for s in shape])
         self.dtype = check_dtype(dtype)
-        self.strides = tuple(int(s) for s in (strides if strides is not None else contiguous_strides(self.shape)))
+        self.strides = tuple([int(s) for s in (strides if strides is not None else contiguous_strides(self.shape))])
         self.offset = int(offset)
         check_extent(storage, self.shape, self.strides, self.offset, self.dtype)
         self.id = next(_ids)
@@ -125,9 +126,17 @@ class HipTensorHandle:
     @classmethod
     def create_new(cls, shape, dtype: str, data=None) -> "HipTensorHandle":
         check_dtype(dtype)
-        n = numel_of(shape)
+        shape = tuple([int(s) for s in shape])
+        n = math.prod(shape)
         storage = HipStorage(n * ITEMSIZE[dtype])
-        h = cls(storage, shape, dtype)
+        if n > 0 and min(shape, default=1) > 0:
+            # a storage of exactly these elements: nothing to check
+            h = cls.__new__(cls)
+            h.storage, h.shape, h.dtype, h.strides, h.offset = storage, shape, dtype, tuple(contiguous_strides(shape)), 0
+            h.id = next(_ids)
+            h._disposed = False
+        else:
+            h = cls(storage, shape, dtype)
         if data is not None:
             arr = to_storage_array(data, dtype).reshape(-1)
             if arr.size != n:
@@ -143,7 +152,7 @@ class HipTensorHandle:
     # -- properties ---------------------------------------------------------------------------
     @property
     def numel(self) -> int:
-        return numel_of(self.shape)
+        return math.prod(self.shape)
 
     @property
     def itemsize(self) -> int:
@@ -163,13 +172,20 @@ class HipTensorHandle:
 
     def data_ptr(self) -> int:
         """Device address of element 0 of this view (storage base + offset)."""
-        if self._disposed or self.storage.is_freed:
+        storage = self.storage
+        if self._disposed or storage._refs <= 0:
             raise RuntimeError(f"tensor {self.id} used after dispose")
-        return self.storage.ptr + self.offset * self.itemsize
+        return storage.ptr + self.offset * ITEMSIZE[self.dtype]
 
     def is_contiguous(self) -> bool:
-        expected = contiguous_strides(self.shape)
-        return all(sz == 1 or st == ex for sz, st, ex in zip(self.shape, self.strides, expected))
+        acc = 1
+        for sz, st in zip(reversed(self.shape), reversed(self.strides)):
+            if sz != 1:
+                if st != acc:
+                    return False
+                if sz > 1:
+                    acc *= sz
+        return True
 
     # -- data -----------------------------------------------------------------------------------
     def data_async(self) -> np.ndarray:
