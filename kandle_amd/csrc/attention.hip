@@ -177,8 +177,10 @@ template <typename T>
 constexpr int dc_kpw() { return sizeof(T) == 2 ? 64 : 32; }
 // Keys per split-K chunk.  Head dim 64 halves the bytes of a key row, so a chunk holds twice the
 // keys and moves the same 64 KiB of K (and of V) per workgroup.
-template <typename T, int DH = 128>
-constexpr int dc_chunk() { return DC_WAVES * dc_kpw<T>() * (128 / DH); }
+// SH = 4: a quarter of the keys, for calls whose chunks of full size would leave CUs idle
+// (decode_shrink).
+template <typename T, int DH = 128, int SH = 1>
+constexpr int dc_chunk() { return DC_WAVES * dc_kpw<T>() * (128 / DH) / SH; }
 
 // Key count of sequence b: seq_lens[b] (or the uniform length when seq_lens is NULL), clamped to
 // [0, max_len] so that a bad device-side length can never index past the cache.
@@ -202,7 +204,7 @@ __device__ __forceinline__ const float2* decode_part_ml(const float* part, int h
   return reinterpret_cast<const float2*>(part + (int64_t)gridDim.z * hq * max_chunks * DH);
 }
 
-template <typename T, int G, int DH = 128>
+template <typename T, int G, int DH = 128, int SH = 1>
 __global__ __launch_bounds__(256) void decode_partial_kernel(const T* __restrict__ Q, const T* __restrict__ K,
                                                              const T* __restrict__ V, const int32_t* __restrict__ lens,
                                                              int uniform_len, int max_len, int hq, int nsub,
@@ -215,9 +217,9 @@ __global__ __launch_bounds__(256) void decode_partial_kernel(const T* __restrict
   constexpr int EPL = 16 / (int)sizeof(T);            // elements per 16-byte load
   constexpr int LPK = D / EPL;                        // lanes per key row (16 bf16, 32 f32 at D = 128)
   constexpr int KPI = 64 / LPK;                       // keys per load instruction (4 bf16, 2 f32 at 128)
-  constexpr int KPW = dc_kpw<T>() * (128 / DH);
-  constexpr int CHUNK = dc_chunk<T, DH>();
-  constexpr int NI = KPW / KPI;                       // load instructions per wave (16)
+  constexpr int KPW = dc_kpw<T>() * (128 / DH) / SH;
+  constexpr int CHUNK = dc_chunk<T, DH, SH>();
+  constexpr int NI = KPW / KPI;                       // load instructions per wave (16 / SH)
   static_assert(DH == 128 || DH == 64, "head dim 64 or 128");
   __shared__ float red_m[DC_WAVES][G];
   __shared__ float red_l[DC_WAVES][G];
@@ -453,7 +455,7 @@ struct Row8 {
 // row p from its own registers and only the first group's writes it).
 // Both decode kernels take G query heads per workgroup; blockIdx.y is the group, and a kv head
 // whose ratio hq / hkv is above 8 (or not a multiple of the G chosen) is served by nsub groups.
-template <typename T, int G, bool FUSE = false, int DH = 128>
+template <typename T, int G, bool FUSE = false, int DH = 128, int SH = 1>
 __global__ __launch_bounds__(256) void decode_partial_rows_kernel(const T* __restrict__ Q, const T* __restrict__ K,
                                                                   const T* __restrict__ V,
                                                                   const int32_t* __restrict__ lens, int uniform_len,
@@ -462,9 +464,9 @@ __global__ __launch_bounds__(256) void decode_partial_rows_kernel(const T* __res
                                                                   float* __restrict__ part, DecodeFuse fz) {
   constexpr bool F32 = sizeof(T) == 4;
   static_assert(DH == 128 || (DH == 64 && !FUSE), "head dim 128, or 64 without the fused block");
-  constexpr int D = DH, LPR = D / 8, NI = F32 ? 8 : 16, KPI = 64 / LPR, KPW = NI * KPI, CHUNK = DC_WAVES * KPW,
+  constexpr int D = DH, LPR = D / 8, NI = (F32 ? 8 : 16) / SH, KPI = 64 / LPR, KPW = NI * KPI, CHUNK = DC_WAVES * KPW,
                 NS = DC_WAVES * KPI;
-  static_assert(CHUNK == dc_chunk<T, DH>(), "chunk size shared with the merge");
+  static_assert(CHUNK == dc_chunk<T, DH, SH>(), "chunk size shared with the merge");
   __shared__ float red_m[NS][G];
   __shared__ float red_l[NS][G];
   __shared__ float red_o[NS][G][D];
@@ -652,7 +654,7 @@ __global__ __launch_bounds__(256) void decode_partial_rows_kernel(const T* __res
 // h.  8 groups of 32 threads (one per column) each run one online log-sum-exp pass over every 8th
 // chunk (running max, denominator and column sum, rescaled when the max grows), and the 8 group
 // states are combined through LDS.  The grid's x extent is DH / 32.
-template <typename T, int DH = 128>
+template <typename T, int DH = 128, int SH = 1>
 __device__ __forceinline__ void decode_merge_cols_body(const float* __restrict__ part, int L, int hq, int max_chunks,
                                                        const AttnStrides& st, T* __restrict__ O) {
   constexpr int D = DH, COLS = 32, NG = 8;
@@ -662,7 +664,7 @@ __device__ __forceinline__ void decode_merge_cols_body(const float* __restrict__
   const int tid = threadIdx.x;
   const int col = tid & (COLS - 1), grp = tid >> 5;
   const int d = cg * COLS + col;
-  const int nch = (L + dc_chunk<T, DH>() - 1) / dc_chunk<T, DH>();
+  const int nch = (L + dc_chunk<T, DH, SH>() - 1) / dc_chunk<T, DH, SH>();
   const int64_t row0 = ((int64_t)b * hq + h) * max_chunks;
   const float* po = decode_part_o(part) + row0 * D + d;
   const float2* pml = decode_part_ml<DH>(part, hq, max_chunks) + row0;
@@ -715,12 +717,12 @@ __device__ __forceinline__ void decode_merge_cols_body(const float* __restrict__
   }
 }
 
-template <typename T, int DH = 128>
+template <typename T, int DH = 128, int SH = 1>
 __global__ __launch_bounds__(256) void decode_merge_cols_kernel(const float* __restrict__ part,
                                                                 const int32_t* __restrict__ lens, int uniform_len,
                                                                 int max_len, int hq, int max_chunks, AttnStrides st,
                                                                 T* __restrict__ O) {
-  decode_merge_cols_body<T, DH>(part, decode_len(lens, uniform_len, blockIdx.z, max_len), hq, max_chunks, st, O);
+  decode_merge_cols_body<T, DH, SH>(part, decode_len(lens, uniform_len, blockIdx.z, max_len), hq, max_chunks, st, O);
 }
 
 // The merge of the fused decode block (one sequence, length *position + 1): the same kernel body
@@ -757,19 +759,6 @@ AttnStrides load_strides(const int64_t* s) {
   return a;
 }
 
-// Bytes of split-K partials launch_decode needs: o rows + (m, l) per (sequence, head, chunk).
-template <typename T, int DH = 128>
-size_t decode_part_bytes(int batch, int hq, int64_t max_len) {
-  const int64_t max_chunks = (max_len + dc_chunk<T, DH>() - 1) / dc_chunk<T, DH>();
-  return (size_t)batch * hq * max_chunks * (DH + 2) * sizeof(float);
-}
-
-size_t decode_part_bytes_for(int dtype, int d, int batch, int hq, int64_t max_len) {
-  if (dtype == KH_BF16)
-    return d == 64 ? decode_part_bytes<uint16_t, 64>(batch, hq, max_len) : decode_part_bytes<uint16_t>(batch, hq, max_len);
-  return d == 64 ? decode_part_bytes<float, 64>(batch, hq, max_len) : decode_part_bytes<float>(batch, hq, max_len);
-}
-
 // Query heads per decode workgroup for GQA ratio G: G itself up to 8, else its largest divisor
 // up to 8 (G / that many workgroups then share each kv head's chunk, each reading its K/V rows).
 inline int decode_group_heads(int G) {
@@ -779,22 +768,46 @@ inline int decode_group_heads(int G) {
   return gc;
 }
 
+// A chunk's workgroup keeps 64 KiB of K and of V in flight, which one CU takes 4-5 us to load; when the
+// cache holds fewer such chunks than two per CU, chunks of a quarter spread the rows over four times the
+// CUs.  Both kernels of a call, 16 / 8 heads, 128: two fp32 sequences of 777 keys 11.5 -> 7.7 us, eight of 700
+// 14.8 -> 11.6, one bf16 of 600 8.4 -> 6.8; one fp32 of 16000 keys (1000 full chunks) 23.9 us either way.
+inline int decode_shrink(int batch, int hq, int hkv, int chunk, int64_t max_len) {
+  const int64_t groups = hq / decode_group_heads(hq / hkv);
+  return (max_len + chunk - 1) / chunk * groups * batch < 2 * 256 ? 4 : 1;
+}
+
+// Bytes of split-K partials launch_decode needs: o rows + (m, l) per (sequence, head, chunk).
+template <typename T, int DH = 128>
+size_t decode_part_bytes(int batch, int hq, int hkv, int64_t max_len) {
+  const int ch = dc_chunk<T, DH>() / decode_shrink(batch, hq, hkv, dc_chunk<T, DH>(), max_len);
+  return (size_t)batch * hq * ((max_len + ch - 1) / ch) * (DH + 2) * sizeof(float);
+}
+
+size_t decode_part_bytes_for(int dtype, int d, int batch, int hq, int hkv, int64_t max_len) {
+  if (dtype == KH_BF16)
+    return d == 64 ? decode_part_bytes<uint16_t, 64>(batch, hq, hkv, max_len)
+                   : decode_part_bytes<uint16_t>(batch, hq, hkv, max_len);
+  return d == 64 ? decode_part_bytes<float, 64>(batch, hq, hkv, max_len)
+                 : decode_part_bytes<float>(batch, hq, hkv, max_len);
+}
+
 // part_in: the partials buffer (at least decode_part_bytes), or nullptr to take one from the
 // caching allocator for the duration of the call.
-template <typename T, int DH = 128>
-int launch_decode(const void* q, const void* k, const void* v, void* o, const int32_t* lens, int uniform_len,
+template <typename T, int DH, int SH>
+int launch_decode_chunks(const void* q, const void* k, const void* v, void* o, const int32_t* lens, int uniform_len,
                   int batch, int hq, int hkv, int64_t max_len, const AttnStrides& st, float scale,
-                  float* part_in = nullptr) {
+                  float* part_in) {
   const int GC = decode_group_heads(hq / hkv), nsub = hq / hkv / GC;
   KH_REQUIRE((int64_t)hkv * nsub <= 65535, "kh_decode_attention: %d query heads need too many workgroup groups", hq);
   const int64_t lim = int64_t(1) << 31;
-  constexpr int CH = dc_chunk<T, DH>();
-  KH_REQUIRE((max_len + CH) * st.ks * (int64_t)sizeof(T) < lim && (max_len + CH) * st.vs * (int64_t)sizeof(T) < lim,
+  constexpr int CH = dc_chunk<T, DH, SH>();
+  KH_REQUIRE((max_len + dc_chunk<T, DH>()) * st.ks * (int64_t)sizeof(T) < lim && (max_len + dc_chunk<T, DH>()) * st.vs * (int64_t)sizeof(T) < lim,
              "kh_decode_attention: one head of the cache spans more than 2 GiB");
   const int ml = (int)max_len;
   const int max_chunks = (ml + CH - 1) / CH;
   KH_REQUIRE(max_chunks <= 65535 * 64, "kh_decode_attention: max_len too large");
-  float* part = part_in ? part_in : (float*)scratch_alloc(decode_part_bytes<T, DH>(batch, hq, max_len));
+  float* part = part_in ? part_in : (float*)scratch_alloc(decode_part_bytes<T, DH>(batch, hq, hkv, max_len));
   if (!part) return KH_ERR_OOM;
   dim3 grid(max_chunks, hkv * nsub, batch);
   const T* Q = (const T*)q;
@@ -804,10 +817,10 @@ int launch_decode(const void* q, const void* k, const void* v, void* o, const in
 #define KH_DECODE_CASE(GG)                                                                                 \
   case GG:                                                                                                 \
     if constexpr (sizeof(T) == 2)                                                                          \
-      decode_partial_rows_kernel<T, GG, false, DH><<<grid, 256, 0, stream()>>>(                            \
+      decode_partial_rows_kernel<T, GG, false, DH, SH><<<grid, 256, 0, stream()>>>(                            \
           Q, K, V, lens, uniform_len, ml, hq, nsub, st, scale, max_chunks, part, DecodeFuse{});            \
     else                                                                                                   \
-      decode_partial_kernel<T, GG, DH><<<grid, 256, 0, stream()>>>(Q, K, V, lens, uniform_len, ml, hq, nsub, st, \
+      decode_partial_kernel<T, GG, DH, SH><<<grid, 256, 0, stream()>>>(Q, K, V, lens, uniform_len, ml, hq, nsub, st, \
                                                                 scale, max_chunks, part);                  \
     break;
   switch (GC) {
@@ -823,7 +836,7 @@ int launch_decode(const void* q, const void* k, const void* v, void* o, const in
 #undef KH_DECODE_CASE
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) {
-    decode_merge_cols_kernel<T, DH><<<dim3(DH / 32, hq, batch), 256, 0, stream()>>>(part, lens, uniform_len, ml,
+    decode_merge_cols_kernel<T, DH, SH><<<dim3(DH / 32, hq, batch), 256, 0, stream()>>>(part, lens, uniform_len, ml,
                                                                                     hq, max_chunks, st, (T*)o);
     e = hipGetLastError();
   }
@@ -834,6 +847,15 @@ int launch_decode(const void* q, const void* k, const void* v, void* o, const in
   }
   KH_DEBUG_SYNC();
   return KH_OK;
+}
+
+template <typename T, int DH = 128>
+int launch_decode(const void* q, const void* k, const void* v, void* o, const int32_t* lens, int uniform_len,
+                  int batch, int hq, int hkv, int64_t max_len, const AttnStrides& st, float scale,
+                  float* part_in = nullptr) {
+  if (decode_shrink(batch, hq, hkv, dc_chunk<T, DH>(), max_len) == 4)
+    return launch_decode_chunks<T, DH, 4>(q, k, v, o, lens, uniform_len, batch, hq, hkv, max_len, st, scale, part_in);
+  return launch_decode_chunks<T, DH, 1>(q, k, v, o, lens, uniform_len, batch, hq, hkv, max_len, st, scale, part_in);
 }
 
 // launch_decode for the element type `dtype` and head dim d (64 or 128).
@@ -1179,7 +1201,7 @@ int kh_decode_attention_noalloc(const void* q, const void* k_cache, const void* 
   if (batch == 0) return KH_OK;
   KH_REQUIRE(batch <= 65535, "kh_decode_attention_noalloc: batch too large");
   KH_REQUIRE(q && k_cache && v_cache && o && seq_lens && strides, "kh_decode_attention_noalloc: null pointer");
-  const size_t need = decode_part_bytes_for(dtype, d, batch, hq, max_len);
+  const size_t need = decode_part_bytes_for(dtype, d, batch, hq, hkv, max_len);
   KH_REQUIRE(need <= kNoAllocScratchBytes,
              "kh_decode_attention_noalloc: batch %d x %d heads x %lld keys needs %zu bytes of split-K partials, "
              "more than the %zu-byte scratch array (use kh_decode_attention)",

@@ -1,0 +1,51 @@
+"""Decode attention's two chunk sizes (kh_decode_attention): full chunks and, where those would leave
+CUs idle, chunks of a quarter."""
+import numpy as np
+import pytest
+
+import oracle
+from kandle_amd import Tensor, synthetic as syn
+from kandle_amd import functional as F
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(seed, shape, dtype):
+    x = syn.normal(seed, shape)
+    if dtype == "float32":
+        return Tensor(x, dtype=dtype), x
+    bits, vals = syn.bf16(x)
+    return Tensor(bits, dtype=dtype), vals
+
+
+@pytest.mark.parametrize("dtype,d,hq", [("float32", 128, 4), ("bfloat16", 128, 4), ("float32", 64, 6), ("bfloat16", 64, 2)])
+def test_quarter_chunks_match_full_chunks_and_oracle(hip, dtype, d, hq):
+    """Lengths on and beside the edges of the small (32 to 128 keys) and full chunks.  The same rows in a
+    cache long enough for two full chunks per CU take full chunks: both against the oracle, and each
+    against the other (fp32: sums of a few hundred products in two groupings, 1e-5 of the largest
+    value; bf16: one output rounding, 2^-8 of it)."""
+    hkv, lens = 2, np.array([0, 1, 31, 32, 33, 127, 128, 129, 300], np.int32)
+    B, short = len(lens), 300
+    full = {("float32", 128): 128, ("bfloat16", 128): 256, ("float32", 64): 256, ("bfloat16", 64): 512}[(dtype, d)]
+    q, qh = _case(1, (B, hq, d), dtype)
+    k, kh = _case(2, (B, hkv, short, d), dtype)
+    v, vh = _case(3, (B, hkv, short, d), dtype)
+    sl = Tensor(lens, dtype="int32")
+    scale = 1.0 / np.sqrt(d)
+    assert (short + full - 1) // full * hkv * B < 512      # quarter chunks
+    got = F.decode_attention(q, k, v, sl, scale).numpy()
+    long = full * (512 // (hkv * B) + 1)                    # (at least 512 full chunks)
+    assert long // full * hkv * B >= 512
+    kl, vl = (F.zeros((B, hkv, long, d), dtype) for _ in range(2))
+    for dst, src in ((kl, k), (vl, v)):
+        F.copy_(F.narrow(dst, 2, 0, short), src)
+    got_full = F.decode_attention(q, kl, vl, sl, scale).numpy()
+    for b, n in enumerate(lens):
+        if n == 0:
+            assert not got[b].any() and not got_full[b].any()
+            continue
+        ref = oracle.sdpa(qh[b][None, :, None], kh[b][None, :, :n], vh[b][None, :, :n], scale=scale)[0, :, 0]
+        bar = np.abs(ref).max() * (1e-4 if dtype == "float32" else 2.0 ** -7)
+        assert np.abs(got[b] - ref).max() <= bar
+        assert np.abs(got_full[b] - ref).max() <= bar
+        assert np.abs(got[b] - got_full[b]).max() <= np.abs(ref).max() * (1e-5 if dtype == "float32" else 2.0 ** -7)
