@@ -769,18 +769,27 @@ inline int decode_group_heads(int G) {
 }
 
 // A chunk's workgroup keeps 64 KiB of K and of V in flight, which one CU takes 4-5 us to load; when the
-// cache holds fewer such chunks than two per CU, chunks of a quarter spread the rows over four times the
-// CUs.  Both kernels of a call, 16 / 8 heads, 128: two fp32 sequences of 777 keys 11.5 -> 7.7 us, eight of 700
-// 14.8 -> 11.6, one bf16 of 600 8.4 -> 6.8; one fp32 of 16000 keys (1000 full chunks) 23.9 us either way.
-inline int decode_shrink(int batch, int hq, int hkv, int chunk, int64_t max_len) {
-  const int64_t groups = hq / decode_group_heads(hq / hkv);
-  return (max_len + chunk - 1) / chunk * groups * batch < 2 * 256 ? 4 : 1;
+// cache holds fewer such chunks than about two per CU, chunks of a quarter spread the rows over four
+// times the CUs.  With more of them it pays as long as the merge has few chunks per sequence.  Both
+// kernels of a call, head dim 128, 16 / 8 heads, full -> quarter chunks: two fp32 sequences of 777 keys
+// 11.5 -> 7.7 us, seven of 1280 17.0 -> 14.5; one bf16 of 600 8.4 -> 6.8, eight of 2100 (9 chunks each)
+// 16.0 -> 13.2; on the other side five bf16 of 3000 (480 chunks, 12 each) 13.2 -> 13.5, one fp32 of 16000
+// 23.8 -> 28.3.  (The quarter chunks' partials stay within the allocation-free entry's scratch.)
+template <typename T, int DH>
+inline int decode_shrink(int batch, int hq, int hkv, int64_t max_len) {
+  constexpr int CH = dc_chunk<T, DH>(), small = dc_chunk<T, DH, 4>();
+  const int64_t per_seq = (max_len + CH - 1) / CH;
+  const int64_t chunks = per_seq * (hq / decode_group_heads(hq / hkv)) * batch;
+  const bool f32 = sizeof(T) == 4;
+  if (!(chunks < (f32 ? 512 : 400) || (chunks < 1200 && per_seq <= (f32 ? 17 : 9)))) return 1;
+  const int64_t bytes = (int64_t)batch * hq * ((max_len + small - 1) / small) * (DH + 2) * (int64_t)sizeof(float);
+  return bytes <= (int64_t)kNoAllocScratchBytes ? 4 : 1;
 }
 
 // Bytes of split-K partials launch_decode needs: o rows + (m, l) per (sequence, head, chunk).
 template <typename T, int DH = 128>
 size_t decode_part_bytes(int batch, int hq, int hkv, int64_t max_len) {
-  const int ch = dc_chunk<T, DH>() / decode_shrink(batch, hq, hkv, dc_chunk<T, DH>(), max_len);
+  const int ch = dc_chunk<T, DH>() / decode_shrink<T, DH>(batch, hq, hkv, max_len);
   return (size_t)batch * hq * ((max_len + ch - 1) / ch) * (DH + 2) * sizeof(float);
 }
 
@@ -853,7 +862,7 @@ template <typename T, int DH = 128>
 int launch_decode(const void* q, const void* k, const void* v, void* o, const int32_t* lens, int uniform_len,
                   int batch, int hq, int hkv, int64_t max_len, const AttnStrides& st, float scale,
                   float* part_in = nullptr) {
-  if (decode_shrink(batch, hq, hkv, dc_chunk<T, DH>(), max_len) == 4)
+  if (decode_shrink<T, DH>(batch, hq, hkv, max_len) == 4)
     return launch_decode_chunks<T, DH, 4>(q, k, v, o, lens, uniform_len, batch, hq, hkv, max_len, st, scale, part_in);
   return launch_decode_chunks<T, DH, 1>(q, k, v, o, lens, uniform_len, batch, hq, hkv, max_len, st, scale, part_in);
 }
