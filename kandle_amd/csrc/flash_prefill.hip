@@ -51,7 +51,8 @@ constexpr bool kPersistXcdLocal = true;  // XCD-local item order where the shape
 constexpr bool kMirrorSlots = true;      // mirrored row slots for the SIMD's second wave
 
 // D: head dimension, 64 or 128.
-template <int BN, int WAVES, int D = 128>
+// BNC_: keys of a compute chunk (64, or 32 in the four-way key-split form).
+template <int BN, int WAVES, int D = 128, int BNC_ = 64>
 struct Cfg {
   static_assert(D == 64 || D == 128, "head_dim 64 or 128");
   static constexpr int THREADS = WAVES * 64;
@@ -71,11 +72,11 @@ struct Cfg {
   static constexpr int NK = BN * CPR / THREADS;      // 16-byte K (and V) chunks per thread per tile
   static constexpr int NQ = D / 16;                  // 16-column MFMA k-steps of q.k (Q registers)
   static constexpr int ND = D / 32;                  // 32-column output tiles of P V
-  // Compute works on 64-key chunks; a staged tile holds NCH of them.
-  static constexpr int BNC = 64;
+  // Compute works on BNC-key chunks; a staged tile holds NCH of them.
+  static constexpr int BNC = BNC_;
   static constexpr int NCH = BN / BNC;
   static constexpr int NSUB = BNC / 32;              // 32-key S^T subtiles per chunk
-  static_assert(BN % BNC == 0, "tiles are whole 64-key chunks");
+  static_assert(BNC % 32 == 0 && BN % BNC == 0, "tiles are whole chunks");
   static_assert(NK >= 1, "tile too small for the workgroup");
 };
 
@@ -115,16 +116,16 @@ __device__ __forceinline__ void mfma_block_begin() { __builtin_amdgcn_s_setprio(
 __device__ __forceinline__ void mfma_block_end() { __builtin_amdgcn_s_setprio(0); }
 
 // Shared per-workgroup setup and staging helpers.
-// KSPLIT = 2 (the persistent kernel's key-split form): waves w and w + WAVES / 2 own the same rows
-// and take the even and the odd 64-key chunk of every tile (key half khalf = w / SW), so an item
-// holds SW / G row slots per query head, half the rows of the KSPLIT = 1 form.
+// KSPLIT = 2, 4 (the persistent kernel's key-split forms): the KSPLIT waves w, w + SW, ... own the same
+// rows and take one chunk of every tile each (key part kpart = w / SW of 64 or, at 4, 32 keys), so an
+// item holds SW / G row slots per query head, 1 / KSPLIT the rows of the KSPLIT = 1 form.
 template <int BN, int WAVES, int D = 128, int KSPLIT = 1>
 struct Flash {
-  using C = Cfg<BN, WAVES, D>;
-  static_assert(KSPLIT == 1 || (KSPLIT == 2 && WAVES == 8 && C::NCH == 2), "key halves: 8 waves, 2 chunks per tile");
+  using C = Cfg<BN, WAVES, D, KSPLIT == 4 ? 32 : 64>;
+  static_assert(KSPLIT == 1 || (WAVES == 8 && C::NCH == KSPLIT), "key parts: 8 waves, a chunk of the tile each");
   static constexpr int SW = WAVES / KSPLIT;  // waves holding an item's row slots
   int G, BMQ, tid, wave, lane, r, g, b, hk, hqi, q0, qw0, qi, ntiles, wave_last_q, wave_tiles, dcol;
-  int khalf = 0, half_last = -1;  // KSPLIT = 2: this wave's key half and its last chunk (-1: none)
+  int kpart = 0, part_last = -1;  // KSPLIT > 1: this wave's key part and its last chunk (-1: none)
   __amdgpu_buffer_rsrc_t rk, rv;
   // Element strides as 32-bit values (the entry checks they fit): half the scalar registers of
   // the 64-bit AttnStrides, which the persistent kernel needs for its item bookkeeping.
@@ -144,7 +145,7 @@ struct Flash {
     r = lane & 31;
     g = lane >> 5;
     dcol = 8 * (tid & (C::CPR - 1));
-    if constexpr (KSPLIT == 2) khalf = wave / SW;
+    if constexpr (KSPLIT > 1) kpart = wave / SW;
   }
   // The wave's row-slot index among the SW waves that hold an item's rows.
   __device__ __forceinline__ int swave() const {
@@ -159,7 +160,7 @@ struct Flash {
   // with a long one.  Only the rows a wave owns change, not any row's arithmetic.
   __device__ __forceinline__ int row_slot(int wpg) const {
     const int i = swave() % wpg;
-    // (KSPLIT = 2: the SIMD's second wave is the other key half of the same slot)
+    // (KSPLIT > 1: the SIMD's second wave is another key part of the same slot)
     if (!kMirrorSlots || WAVES != 8 || KSPLIT != 1 || wave < 4 || wpg == 1) return i;
     return wpg == 8 ? 11 - i : wpg - 1 - i;
   }
@@ -176,11 +177,12 @@ struct Flash {
     qi = qw0 + r;
     const int kv_end = causal ? min(lk, q0 + BMQ) : lk;
     ntiles = (kv_end + BN - 1) / BN;
-    // wave_tiles counts 64-key compute chunks (C::BNC)
+    // wave_tiles counts compute chunks (C::BNC keys)
     const int nchunks = (kv_end + C::BNC - 1) / C::BNC;
     wave_last_q = min(qw0 + 31, lq - 1);
     wave_tiles = qw0 >= lq ? 0 : (causal ? min(nchunks, wave_last_q / C::BNC + 1) : nchunks);
-    if constexpr (KSPLIT == 2) half_last = wave_tiles > khalf ? khalf + 2 * ((wave_tiles - 1 - khalf) / 2) : -1;
+    if constexpr (KSPLIT > 1)
+      part_last = wave_tiles > kpart ? kpart + KSPLIT * ((wave_tiles - 1 - kpart) / KSPLIT) : -1;
     const int hkr = hk / kvsub;
     rk = make_rsrc(K + (int64_t)b * st.kb + (int64_t)hkr * st.kh, (uint32_t)(((int64_t)(lk - 1) * st.ks + D) * 2));
     rv = make_rsrc(V + (int64_t)b * st.vb + (int64_t)hkr * st.vh, (uint32_t)(((int64_t)(lk - 1) * st.vs + D) * 2));
@@ -278,7 +280,7 @@ struct Flash {
     sched_reads_ahead<C::ND * KC, 2>();
     mfma_block_end();
   }
-  // S^T subtiles of one 64-key chunk in LDS; the accumulators start at cinit (INIT) or 0.
+  // S^T subtiles of one compute chunk in LDS; the accumulators start at cinit (INIT) or 0.
   template <bool INIT>
   __device__ __forceinline__ void qk(const uint16_t* ks, const bf16x8 (&qreg)[C::NQ], const f32x16& cinit,
                                      f32x16 (&sacc)[C::NSUB]) const {
@@ -309,7 +311,7 @@ struct Flash {
   // Causal / length mask of chunk t (only chunks crossing the diagonal or the sequence end).
   template <bool CAUSAL>
   __device__ __forceinline__ void mask(int t, int lk, f32x16 (&sc)[C::NSUB]) const {
-    const int kt = t * C::BNC;  // t counts 64-key compute chunks
+    const int kt = t * C::BNC;  // t counts compute chunks
     if ((kt + C::BNC > lk) || (CAUSAL && kt + C::BNC - 1 > qw0)) {
       const int lim = (CAUSAL ? min(lk, qi + 1) : lk) - kt - 8 * g;
 #pragma unroll
@@ -600,7 +602,7 @@ __global__ __launch_bounds__(WAVES * 64, MINB) void flash_fwd_kernel(
     const uint16_t* ks = smem + (t & 1) * STAGE;
 #pragma unroll
     for (int c = 0; c < C::NCH; ++c) {
-      const int tc = t * C::NCH + c;  // 64-key compute chunk
+      const int tc = t * C::NCH + c;  // compute chunk
       if (tc < F.wave_tiles) {
         f32x16 sacc[C::NSUB];
         bf16x8 pk[2 * C::NSUB];
@@ -645,10 +647,10 @@ __global__ __launch_bounds__(WAVES * 64, MINB) void flash_fwd_kernel(
 // each).  When P is a multiple of the pair count, the odd passes are mirrored so that a workgroup
 // keeps one (batch, kv head) pair for all its items (its K/V stay in its XCD's L2).  The per-item
 // arithmetic is the tile kernel's, so outputs are identical to it.
-// KSPLIT = 2 (one sequence of a few thousand tokens: too few 128-row items to pair): items of half
-// the rows, each row slot held by two waves that take the even and the odd 64-key chunk of every
-// tile; at the end of an item the two halves' (m, l, O) merge through the staging buffer the loop
-// left free, and the first half stores the rows.  Its sums are grouped differently from the
+// KSPLIT = 2, 4 (one sequence of up to a few thousand tokens: too few 128-row items to pair): items
+// of a half or a quarter of the rows, each row slot held by two or four waves that take one chunk of
+// every tile each; at the end of an item the parts' (m, l, O) merge pairwise through the staging buffer
+// the loop left free, and the first part stores the rows.  Its sums are grouped differently from the
 // KSPLIT = 1 form, so its outputs differ from it within the rounding of the split.
 // GROUPS: hkv counts groups of G query heads, kvsub of them per real kv head (a GQA ratio other than
 // 1, 2, 4, 8, as the tile kernel's kvsub); without it kvsub is ignored.
@@ -658,8 +660,8 @@ __global__ __launch_bounds__(kPersistWaves * 64, 1) void flash_fwd_persistent_ke
     uint16_t* __restrict__ O, int batch, int hq, int hkv, int lq, int lk, AttnStrides st, float scale, int n_qblocks,
     int kvsub) {
   constexpr int BN = 128, WAVES = kPersistWaves;
-  using C = Cfg<BN, WAVES, D>;
   using FL = Flash<BN, WAVES, D, KSPLIT>;
+  using C = typename FL::C;
   constexpr int STAGE = C::KTILE + C::VTILE;
   __shared__ __attribute__((aligned(16))) uint16_t smem[2 * STAGE];
   const int P = gridDim.x, w = blockIdx.x;
@@ -715,7 +717,7 @@ __global__ __launch_bounds__(kPersistWaves * 64, 1) void flash_fwd_persistent_ke
     const bool more = item(k + 1, bhn, qbn);
     // A wave's Q registers are free once it has formed its last chunk's scores: the next item's Q
     // is loaded into them there (at the start for a wave with no rows in this item).
-    if (more && (KSPLIT == 1 ? F.wave_tiles == 0 : F.half_last < 0)) F.load_q_of(bhn, qbn, hkv, Q, lq, qreg);
+    if (more && (KSPLIT == 1 ? F.wave_tiles == 0 : F.part_last < 0)) F.load_q_of(bhn, qbn, hkv, Q, lq, qreg);
     const int ntiles = F.ntiles;
     for (int t = 0; t < ntiles; ++t) {
       const bool next_same = t + 1 < ntiles;
@@ -731,12 +733,12 @@ __global__ __launch_bounds__(kPersistWaves * 64, 1) void flash_fwd_persistent_ke
       const uint16_t* ks = smem + buf * STAGE;
 #pragma unroll
       for (int c = 0; c < C::NCH; ++c) {
-        const int tc = t * C::NCH + c;  // 64-key compute chunk
-        if (tc < F.wave_tiles && (KSPLIT == 1 || c == F.khalf)) {
+        const int tc = t * C::NCH + c;  // compute chunk
+        if (tc < F.wave_tiles && (KSPLIT == 1 || c == F.kpart)) {
           f32x16 sacc[C::NSUB];
           bf16x8 pk[2 * C::NSUB];
           F.template qk<true>(ks + c * C::BNC * C::KSTR, qreg, sl.mneg, sacc);
-          if (more && tc == (KSPLIT == 1 ? F.wave_tiles - 1 : F.half_last)) F.load_q_of(bhn, qbn, hkv, Q, lq, qreg);
+          if (more && tc == (KSPLIT == 1 ? F.wave_tiles - 1 : F.part_last)) F.load_q_of(bhn, qbn, hkv, Q, lq, qreg);
           F.template mask<CAUSAL>(tc, lk, sacc);
           float ps = SoftmaxLog2::exponentiate(sacc, c2, pk);
           if (sl.need_raise(ps)) {
@@ -758,34 +760,41 @@ __global__ __launch_bounds__(kPersistWaves * 64, 1) void flash_fwd_persistent_ke
     if constexpr (KSPLIT == 1) {
       F.template store_o<false>(O, lq, sl.l, oacc);
     } else {
-      // Merge the two key halves of each row slot: the second writes (m, l, O) per lane into the
-      // free staging buffer (the other holds the next item's first tile), the first combines them
-      // with the log-sum-exp rule and stores the rows.  The last barrier keeps the buffer until
-      // every read is done: the next item's second tile is staged there.
+      // Merge the key parts of each row slot, the upper half of them into the lower until one is left:
+      // a wave of the upper half writes (m, l, O) per lane into the free staging buffer (the other
+      // holds the next item's first tile), its partner combines them with the log-sum-exp rule, and the
+      // first part stores the rows.  The last barrier keeps the buffer until every read is done: the
+      // next item's second tile is staged there.
       constexpr int MS = 2 + 16 * C::ND;  // floats per lane
       static_assert(WAVES / 2 * MS * 64 * 4 <= STAGE * 2, "the merge fits a staging buffer");
-      float* mp = reinterpret_cast<float*>(smem + (buf ^ 1) * STAGE) + F.swave() * MS * 64 + F.lane;
-      if (F.khalf == 1) {
-        mp[0] = sl.m;
-        mp[64] = sl.l;
+      float* mbase = reinterpret_cast<float*>(smem + (buf ^ 1) * STAGE) + F.lane;
+      for (int half = KSPLIT / 2; half >= 1; half /= 2) {
+        if (half < KSPLIT / 2) __syncthreads();
+        float* mp = mbase + ((F.kpart % half) * FL::SW + F.swave()) * MS * 64;
+        if (F.kpart >= half && F.kpart < 2 * half) {
+          mp[0] = sl.m;
+          mp[64] = sl.l;
 #pragma unroll
-        for (int dt = 0; dt < C::ND; ++dt)
+          for (int dt = 0; dt < C::ND; ++dt)
 #pragma unroll
-          for (int j = 0; j < 16; ++j) mp[(2 + 16 * dt + j) * 64] = oacc[dt][j];
+            for (int j = 0; j < 16; ++j) mp[(2 + 16 * dt + j) * 64] = oacc[dt][j];
+        }
+        __syncthreads();
+        if (F.kpart < half) {
+          const float m1 = mp[0], l1 = mp[64];
+          const float mt = fmaxf(sl.m, m1);
+          // a part with no unmasked key has m = -inf and adds nothing (its l and O are 0)
+          const float a0 = sl.m == -INFINITY ? 0.f : fast_exp2((sl.m - mt) * c2);
+          const float a1 = m1 == -INFINITY ? 0.f : fast_exp2((m1 - mt) * c2);
+#pragma unroll
+          for (int dt = 0; dt < C::ND; ++dt)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) oacc[dt][j] = oacc[dt][j] * a0 + mp[(2 + 16 * dt + j) * 64] * a1;
+          sl.l = sl.l * a0 + l1 * a1;
+          sl.m = mt;
+        }
       }
-      __syncthreads();
-      if (F.khalf == 0) {
-        const float m1 = mp[0], l1 = mp[64];
-        const float mt = fmaxf(sl.m, m1);
-        // a half with no unmasked key has m = -inf and adds nothing (its l and O are 0)
-        const float a0 = sl.m == -INFINITY ? 0.f : fast_exp2((sl.m - mt) * c2);
-        const float a1 = m1 == -INFINITY ? 0.f : fast_exp2((m1 - mt) * c2);
-#pragma unroll
-        for (int dt = 0; dt < C::ND; ++dt)
-#pragma unroll
-          for (int j = 0; j < 16; ++j) oacc[dt][j] = oacc[dt][j] * a0 + mp[(2 + 16 * dt + j) * 64] * a1;
-        F.template store_o<false>(O, lq, sl.l * a0 + l1 * a1, oacc);
-      }
+      if (F.kpart == 0) F.template store_o<false>(O, lq, sl.l, oacc);
       __syncthreads();
     }
     if (!more) break;
@@ -808,6 +817,192 @@ constexpr int kWaves = 8;  // waves per workgroup: query rows of 32 * 8 / G, one
 // measured the same as 128-key ones.
 constexpr int kSmallGrid = 256;
 constexpr int kSmallBN = 128;
+
+// =============================================================================================
+// Short calls: no shared tiles.
+// =============================================================================================
+// A workgroup is (batch, query head, 32 queries) with four waves; wave w takes the block's 32-key chunks
+// w, w + 4, ... and loads each chunk's operands straight into registers in the MFMA layouts (K as
+// flash_split_kernel does; V: row m of output tile dt is column ND m + dt, so a lane loads ND consecutive
+// bf16 of each of its 8 keys per 16-key step and picks a tile's operand out of them with byte permutes),
+// the next chunk's K once QK^T has consumed the current one and the next V once PV has.  The four waves'
+// (m, l, O) are merged through LDS in wave order.
+// Short calls are bound by latency: the tile kernels load, store to LDS, cross a barrier and read back
+// for every 128 keys, and a few dozen query blocks leave most CUs idle; here a block's chain is a
+// quarter of its 32-key chunks and no wave waits for another.  Each wave reads its own K and V from L2,
+// though (16 KiB per chunk at head dim 128, about 9.5 TB/s over the chip), which bounds longer calls:
+// hence the limit on the number of chunks.  One sequence, 16 / 8 heads, head dim 128, causal, against the
+// forms below: S = 64 7.5 -> 5.8 us, 256 11.5 -> 8.0, 480 16.9 -> 10.5; S = 1024 24.2 -> 27.5 (8448 chunks).
+// The limit of 2048 chunks keeps 512-token prompts of 16 heads (2176 chunks, 17.7 -> 10.9) on the forms
+// below: their sums decide the bf16 model's logits to the last few percent of the tolerance its parity
+// test allows, and either grouping of the chunks here was over it (0.0201 and 0.0203 of 0.02; 0.0194
+// there).  Without the causal mask the chains are equal and short calls of many
+// blocks stay on the tile kernels (eight sequences of 128, 512 blocks: 8.7 us there, 9.5 here).
+constexpr int kDirectWaves = 4;
+constexpr int64_t kDirectChunks = 2048;
+using FL128 = Flash<128, 8, 128>;  // for its swap23 and 32-bit strides
+using Strides32 = FL128::Strides32;
+
+template <bool CAUSAL, int D>
+__global__ __launch_bounds__(kDirectWaves * 64, 2) void flash_direct_kernel(
+    const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V,
+    uint16_t* __restrict__ O, int hq, int ratio, int lq, int lk, Strides32 st, float scale, int n_qblocks) {
+  constexpr int NQ = D / 16, ND = D / 32;
+  using VRow = std::conditional_t<ND == 4, uint2, uint32_t>;  // ND consecutive bf16 of a V row
+  __shared__ __attribute__((aligned(16))) float part[(kDirectWaves - 1) * (2 + 16 * ND) * 64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, r = lane & 31, g = lane >> 5;
+  // As flash_split_kernel: an XCD runs whole query heads where the grid divides by 8, heaviest block first.
+  int logical = blockIdx.x;
+  if (gridDim.x % kXcds == 0) logical = (blockIdx.x % kXcds) * (gridDim.x / kXcds) + blockIdx.x / kXcds;
+  const int qblk = n_qblocks - 1 - logical % n_qblocks, bh = logical / n_qblocks;
+  const int b = bh / hq, h = bh % hq, hk = h / ratio;
+  const int q0 = qblk * 32, qi = q0 + r;
+  const int kv_end = CAUSAL ? min(lk, q0 + 32) : lk;
+  const int nchunks = (kv_end + 31) / 32;
+  const float c2 = scale * kLog2e;
+
+  const auto rk = make_rsrc(K + (int64_t)b * st.kb + (int64_t)hk * st.kh, (uint32_t)(((int64_t)(lk - 1) * st.ks + D) * 2));
+  const auto rv = make_rsrc(V + (int64_t)b * st.vb + (int64_t)hk * st.vh, (uint32_t)(((int64_t)(lk - 1) * st.vs + D) * 2));
+  const int krow = FL128::swap23(r);
+  uint4 kr[NQ];
+  VRow vr[16];
+  auto load_k = [&](int tc) {
+    const uint32_t ko = (uint32_t)((32 * tc + krow) * st.ks + 8 * g) * 2u;
+#pragma unroll
+    for (int c = 0; c < NQ; ++c) kr[c] = buf_load16(rk, ko + 32 * c);
+  };
+  auto load_v = [&](int tc) {
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t vo = (uint32_t)((32 * tc + 16 * kc + 8 * g + e) * st.vs + ND * r) * 2u;
+        if constexpr (ND == 4)
+          vr[8 * kc + e] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rv, vo, 0, 0));
+        else
+          vr[8 * kc + e] = __builtin_amdgcn_raw_buffer_load_b32(rv, vo, 0, 0);
+      }
+  };
+  int tc = wave;
+  if (tc < nchunks) {
+    load_k(tc);
+    load_v(tc);
+  }
+  bf16x8 qreg[NQ];
+  {
+    const auto rq = make_rsrc(Q + (int64_t)b * st.qb + (int64_t)h * st.qh, (uint32_t)(((int64_t)(lq - 1) * st.qs + D) * 2));
+    const uint32_t qoff = (uint32_t)(qi * st.qs + 8 * g) * 2u;
+#pragma unroll
+    for (int c = 0; c < NQ; ++c) qreg[c] = as_bf16x8(buf_load16(rq, qoff + 32 * c));
+  }
+  f32x16 oacc[ND];
+#pragma unroll
+  for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) oacc[dt][j] = 0.f;
+  SoftmaxLog2 sl;
+  // Word w of a V row's load, and the half of it that tile dt's column sits in.
+  auto word_of = [](const VRow& v, int w) -> uint32_t {
+    if constexpr (ND == 4)
+      return w == 0 ? v.x : v.y;
+    else
+      return v;
+  };
+#pragma unroll 1
+  for (; tc < nchunks; tc += kDirectWaves) {
+    f32x16 sacc[1];
+    sacc[0] = sl.mneg;
+#pragma unroll
+    for (int c = 0; c < NQ; ++c)
+      sacc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(kr[c]), qreg[c], sacc[0], 0, 0, 0);
+    const bool more = tc + kDirectWaves < nchunks;
+    if (more) load_k(tc + kDirectWaves);
+    // causal / length mask (keys 32 tc + 8 g + (j & 7) + 16 (j >> 3) of this lane)
+    const int kb = 32 * tc;
+    if (kb + 32 > lk || (CAUSAL && kb + 31 > q0)) {
+      const int lim = (CAUSAL ? min(lk, qi + 1) : lk) - kb - 8 * g;
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        if (16 * (j >> 3) + (j & 7) >= lim) sacc[0][j] = -INFINITY;
+    }
+    bf16x8 pk[2];
+    float ps = SoftmaxLog2::exponentiate(sacc, c2, pk);
+    if (sl.need_raise(ps)) {
+      sl.raise(sacc, c2, oacc);
+      ps = SoftmaxLog2::exponentiate(sacc, c2, pk);
+    }
+    sl.l += ps;
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+      for (int kc = 0; kc < 2; ++kc) {
+        const VRow* v = vr + 8 * kc;
+        const uint32_t sel = (dt & 1) ? 0x07060302u : 0x05040100u;  // high or low halves of two words
+        uint4 a;
+        a.x = __builtin_amdgcn_perm(word_of(v[1], dt >> 1), word_of(v[0], dt >> 1), sel);
+        a.y = __builtin_amdgcn_perm(word_of(v[3], dt >> 1), word_of(v[2], dt >> 1), sel);
+        a.z = __builtin_amdgcn_perm(word_of(v[5], dt >> 1), word_of(v[4], dt >> 1), sel);
+        a.w = __builtin_amdgcn_perm(word_of(v[7], dt >> 1), word_of(v[6], dt >> 1), sel);
+        oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), pk[kc], oacc[dt], 0, 0, 0);
+      }
+    if (more) load_v(tc + kDirectWaves);
+  }
+  // Merge: waves 1..3 write (m, l, O) to LDS; wave 0 combines them in wave order and stores the rows.
+  constexpr int MS = (2 + 16 * ND) * 64;
+  float l = sl.l;
+  if (wave > 0) {
+    float* p = part + (wave - 1) * MS + lane;
+    p[0] = sl.m;
+    p[64] = l;
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) p[(2 + 16 * dt + j) * 64] = oacc[dt][j];
+  }
+  __syncthreads();
+  if (wave > 0) return;
+  float mo[kDirectWaves], mt = sl.m;
+  mo[0] = sl.m;
+#pragma unroll
+  for (int w2 = 1; w2 < kDirectWaves; ++w2) {
+    mo[w2] = part[(w2 - 1) * MS + lane];
+    mt = fmaxf(mt, mo[w2]);
+  }
+  // a wave with no unmasked key has m = -inf and adds nothing (its l and O are 0)
+  const float a0 = mo[0] == -INFINITY ? 0.f : fast_exp2((mo[0] - mt) * c2);
+  l *= a0;
+#pragma unroll
+  for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) oacc[dt][j] *= a0;
+#pragma unroll
+  for (int w2 = 1; w2 < kDirectWaves; ++w2) {
+    const float* p = part + (w2 - 1) * MS + lane;
+    const float a = mo[w2] == -INFINITY ? 0.f : fast_exp2((mo[w2] - mt) * c2);
+    l += a * p[64];
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) oacc[dt][j] += a * p[(2 + 16 * dt + j) * 64];
+  }
+  // Register j = 4 a + i of tile dt holds A row m = 8 a + 4 g + i, i.e. d = ND m + dt: the tiles'
+  // registers j are consecutive outputs.
+  const float l_tot = l + __shfl_xor(l, 32, 64);
+  if (qi < lq) {
+    const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
+    uint16_t* orow = O + (int64_t)b * st.ob + (int64_t)h * st.oh + (int64_t)qi * st.os;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int m = 8 * (j >> 2) + 4 * g + (j & 3);
+      const uint32_t w0 = pack_bf16x2(oacc[0][j] * inv, oacc[1][j] * inv);
+      if constexpr (ND == 4)
+        *reinterpret_cast<uint2*>(orow + 4 * m) = make_uint2(w0, pack_bf16x2(oacc[ND - 2][j] * inv, oacc[ND - 1][j] * inv));
+      else
+        *reinterpret_cast<uint32_t*>(orow + 2 * m) = w0;
+    }
+  }
+}
 
 // hkv here counts groups of hq / hkv query heads sharing K/V tiles; with kvsub > 1 they are
 // sub-groups, kvsub of them per real kv head (see prefill_groups).
@@ -844,27 +1039,78 @@ int launch_prefill_d(const void* q, const void* k, const void* v, void* o, int b
   const int64_t nblk64 = (int64_t)nqb * batch * hkv;
   KH_REQUIRE(nblk64 <= INT32_MAX, "kh_flash_attention: grid too large");
   // The persistent forms (one resident workgroup per CU); GROUPS instantiations serve kvsub > 1.
-  auto persist = [&](auto ksplit, int n_qb) {
+  auto persist = [&](auto causal_c, auto ksplit, int n_qb) {
     constexpr int KSP = decltype(ksplit)::value;
+    constexpr bool CS = decltype(causal_c)::value;
     if (kvsub > 1)
-      flash_fwd_persistent_kernel<true, D, KSP, true><<<cu_count(), kPersistWaves * 64, 0, stream()>>>(
+      flash_fwd_persistent_kernel<CS, D, KSP, true><<<cu_count(), kPersistWaves * 64, 0, stream()>>>(
           (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o, batch, hq, hkv, (int)lq, (int)lk,
           st, scale, n_qb, kvsub);
     else
-      flash_fwd_persistent_kernel<true, D, KSP, false><<<cu_count(), kPersistWaves * 64, 0, stream()>>>(
+      flash_fwd_persistent_kernel<CS, D, KSP, false><<<cu_count(), kPersistWaves * 64, 0, stream()>>>(
           (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o, batch, hq, hkv, (int)lq, (int)lk,
           st, scale, n_qb, 1);
   };
+  // Short calls: (32 queries x 32 keys) blocks per query head up to kDirectChunks in all.
+  const int64_t nq32 = (lq + 31) / 32, nk32 = (lk + 31) / 32, full = nq32 < nk32 ? nq32 : nk32;
+  const int64_t per_head = causal ? full * (full + 1) / 2 + (nq32 - full) * nk32 : nq32 * nk32;
+  if (per_head * batch * hq * D <= kDirectChunks * 128 && (causal || nq32 * batch * hq <= 448)) {
+    const Strides32 s32{(int32_t)st.qb, (int32_t)st.qh, (int32_t)st.qs, (int32_t)st.kb, (int32_t)st.kh, (int32_t)st.ks,
+                        (int32_t)st.vb, (int32_t)st.vh, (int32_t)st.vs, (int32_t)st.ob, (int32_t)st.oh, (int32_t)st.os};
+    const int grid = (int)(nq32 * batch * hq), ratio = hq / hkv_real;
+    const uint16_t *Q = (const uint16_t*)q, *K = (const uint16_t*)k, *V = (const uint16_t*)v;
+    if (causal)
+      flash_direct_kernel<true, D><<<grid, kDirectWaves * 64, 0, stream()>>>(Q, K, V, (uint16_t*)o, hq, ratio, lq, lk,
+                                                                            s32, scale, (int)nq32);
+    else
+      flash_direct_kernel<false, D><<<grid, kDirectWaves * 64, 0, stream()>>>(Q, K, V, (uint16_t*)o, hq, ratio, lq, lk,
+                                                                             s32, scale, (int)nq32);
+    KH_CHECK_LAUNCH();
+    return KH_OK;
+  }
   if (causal && G <= 4 && kPersistMinItems > 0 && nblk64 < (int64_t)kPersistMinItems * cu_count()) {
     // Too few 128-row items to pair heavy with light ones (one sequence of a few thousand tokens:
     // 256 items of very unequal length on 256 CUs): the key-split persistent form, whose items
     // hold half the rows, when that gives at least half the CUs one (B = 1, 16 / 8 heads: S = 4096
     // 117.6 -> 103.0 us, 2048 63.4 -> 42.1, 1024 30.1 -> 24.6; shorter prompts keep the small
     // workgroups below).
+    // (groups of one or two query heads) a quarter of the rows, where that makes at most one and a half
+    // items per CU and more than one per two CUs: S = 1024 24.1 -> 21.0 us, 1531 31.0 -> 27.8; 2048 (two per CU) 38.5 either way, and
+    // two sequences of 1500 (three) 33 -> 49.
+    if (G <= 2) {
+      const int rows4 = 32 * (kPersistWaves / 4 / G), nqb4 = (lq + rows4 - 1) / rows4;
+      const int64_t items4 = (int64_t)nqb4 * batch * hkv;
+      if (2 * items4 > cu_count() && 2 * items4 <= 3 * cu_count()) {
+        persist(std::true_type{}, std::integral_constant<int, 4>{}, nqb4);
+        KH_CHECK_LAUNCH();
+        return KH_OK;
+      }
+    }
     const int BMQ2 = 32 * (kPersistWaves / 2 / G);
     const int nqb2 = (lq + BMQ2 - 1) / BMQ2;
     if ((int64_t)nqb2 * batch * hkv >= cu_count() / 2) {
-      persist(std::integral_constant<int, 2>{}, nqb2);
+      persist(std::true_type{}, std::integral_constant<int, 2>{}, nqb2);
+      KH_CHECK_LAUNCH();
+      return KH_OK;
+    }
+  }
+  if (!causal && G <= 4 && nblk64 < kSmallGrid && lk > 256) {
+    // Few equal items: the key-split form with the fewest tile times (one of the form split in two takes
+    // about 1.2 of those of the form split in four, for twice the rows), if the items fill half the chip
+    // and have a few tiles to share out.  16 / 8 heads, against the workgroups below: one sequence of 1024
+    // 29.1 -> 22.1 us, 1531 79.2 -> 32.4, 2600 193 -> 92; four of 300 25.4 -> 15.1; eight of 128 (one tile)
+    // 8.8 there, 10.8 here.
+    const int rows2 = 32 * (kPersistWaves / 2 / G), nqb2 = (lq + rows2 - 1) / rows2;
+    const int64_t cu = cu_count(), items2 = (int64_t)nqb2 * batch * hkv;
+    const int rows4 = G <= 2 ? 32 * (kPersistWaves / 4 / G) : rows2, nqb4 = (lq + rows4 - 1) / rows4;
+    const int64_t items4 = (int64_t)nqb4 * batch * hkv;
+    if (G <= 2 && items4 >= cu / 2 && 5 * ((items4 + cu - 1) / cu) <= 6 * ((items2 + cu - 1) / cu)) {
+      persist(std::false_type{}, std::integral_constant<int, 4>{}, nqb4);
+      KH_CHECK_LAUNCH();
+      return KH_OK;
+    }
+    if (items2 >= cu / 2) {
+      persist(std::false_type{}, std::integral_constant<int, 2>{}, nqb2);
       KH_CHECK_LAUNCH();
       return KH_OK;
     }
@@ -882,7 +1128,7 @@ int launch_prefill_d(const void* q, const void* k, const void* v, void* o, int b
   } else if (causal && kPersistMinItems > 0 && nblk64 >= (int64_t)kPersistMinItems * cu_count()) {
     // Enough causal query blocks for every CU to take several: one resident workgroup per CU.
     static_assert(kPersistWaves == kWaves, "the persistent kernel's query blocks are the tile kernel's");
-    persist(std::integral_constant<int, 1>{}, nqb);
+    persist(std::true_type{}, std::integral_constant<int, 1>{}, nqb);
   } else if (causal) {
     launch_fwd<128, kWaves, true, D>(q, k, v, o, batch, hq, hkv, lq, lk, st, scale, kvsub);
   } else {
@@ -927,8 +1173,6 @@ int launch_prefill_d(const void* q, const void* k, const void* v, void* o, int b
 // in a separate launch, so that the attention loop only loads ready operands -- C1 13.3 -> 20.2 us
 // and C5's prefill 3.23 -> 3.42 ms: the extra dependent launch costs more than the conversion.
 constexpr int kSplitWaves = 4;
-using FL128 = Flash<128, 8, 128>;  // for its swap23 and 32-bit strides
-using SplitStrides = FL128::Strides32;
 
 // Four floats -> their bf16 hi parts and the bf16 of the remainders, as two 8-byte rows.
 __device__ __forceinline__ void split4(const uint4& x, uint2& hi, uint2& lo) {
@@ -967,7 +1211,7 @@ __device__ __forceinline__ uint32_t word(const uint4& u) {
 template <bool CAUSAL>
 __global__ __launch_bounds__(kSplitWaves * 64, 1) void flash_split_kernel(
     const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V, float* __restrict__ O,
-    int hq, int ratio, int lq, int lk, SplitStrides st, float scale, int n_qblocks) {
+    int hq, int ratio, int lq, int lk, Strides32 st, float scale, int n_qblocks) {
   constexpr int D = 128, NQ = D / 16, ND = D / 32;
   __shared__ __attribute__((aligned(16))) float part[(kSplitWaves - 1) * 66 * 64];  // [wave - 1][66][lane]
   const int tid = threadIdx.x;
@@ -1207,7 +1451,7 @@ int launch_flash_split_f32(const void* q, const void* k, const void* v, void* o,
   const int nqb = (lq + 31) / 32;
   const int64_t grid = (int64_t)nqb * batch * hq;
   KH_REQUIRE(grid <= INT32_MAX, "kh_flash_attention_split: grid too large");
-  const SplitStrides s32{(int32_t)st.qb, (int32_t)st.qh, (int32_t)st.qs, (int32_t)st.kb, (int32_t)st.kh, (int32_t)st.ks,
+  const Strides32 s32{(int32_t)st.qb, (int32_t)st.qh, (int32_t)st.qs, (int32_t)st.kb, (int32_t)st.kh, (int32_t)st.ks,
                          (int32_t)st.vb, (int32_t)st.vh, (int32_t)st.vs, (int32_t)st.ob, (int32_t)st.oh, (int32_t)st.os};
   const float *Q = (const float*)q, *K = (const float*)k, *V = (const float*)v;
   float* O = (float*)o;
