@@ -408,7 +408,7 @@ int kh_gemm_swiglu(const void* x, int64_t ldx, const void* w_gu, int64_t ldw, vo
  * must be 128; operands 16-byte aligned; k, ldx, ldw multiples of 8.  The [M, (hq + 2 hkv) * 128]
  * projection output is never written.  Each output sums over all of k: the values kh_gemm followed
  * by kh_qk_norm_rope produce whenever kh_gemm runs its MFMA tiles unsplit (M > 8 and
- * kh_gemm_split_count() == 1).  Fuses GroupedQueryAttention's q/k/v projections with
+ * kh_gemm_split_count_for() == 1).  Fuses GroupedQueryAttention's q/k/v projections with
  * q_norm / k_norm, RoPE and the cache update (reference: packages/model-utils/src/attention/
  * gqa.ts:269-309; rope.ts:546-644; kv-cache.ts:164-212); no single reference kernel. */
 int kh_gemm_qk_norm_rope(const void* x, int64_t ldx, const void* w_qkv, int64_t ldw, int64_t n_batch,
@@ -433,16 +433,19 @@ int kh_gemm_qk_norm_rope_table(const void* x, int64_t ldx, const void* w_qkv, in
  * QKV projection (kh_gemm_qk_norm_rope_table). */
 int kh_rope_table(const int32_t* positions, int64_t n, const float* inv_freq, int half, float* out);
 
-/* The split count kh_gemm uses for a [m, k] x [n, k]^T product with bf16 weights and contiguous,
- * 16-byte aligned operands, whether A is bf16 or fp32 (1: not split).  A caller that splits the same product with
- * kh_gemm_splitk_partials and adds the partials in split order reproduces kh_gemm bit for bit. */
+/* The split count kh_gemm uses for a bf16 [m, k] x [n, k]^T product with contiguous, 16-byte aligned
+ * operands (1: not split).  A caller that splits the same product with kh_gemm_splitk_partials and
+ * adds the partials in split order reproduces kh_gemm bit for bit. */
 int kh_gemm_split_count(int64_t m, int64_t n, int64_t k, int* splits);
+
+/* The same for an A of type a_dtype (KH_BF16 or KH_F32) and bf16 weights (kh_gemm_ex). */
+int kh_gemm_split_count_for(int64_t m, int64_t n, int64_t k, int a_dtype, int* splits);
 
 /* The split-K stage of kh_gemm alone: part[s][i][j] (fp32, s < splits, row-major [m, n], split s
  * at part + s*m*n) = the sum over split s's k range of a[i, :] * b[j, :] (bf16 a [m, k] with row
  * stride lda -- or fp32 a with a_dtype KH_F32, split as kh_gemm_ex does -- and b [n, k] with row
  * stride ldb), k ranges of ceil(k / splits) rounded up to 128.
- * splits must equal kh_gemm_split_count's count for this shape (and the operands meet the MFMA
+ * splits must equal kh_gemm_split_count_for's count for this shape, or the other A type's (and the operands meet the MFMA
  * path's alignment: 16-byte aligned, k, lda, ldb multiples of 8).  The producer half of the
  * projection + residual + RMSNorm fusion below (no reference counterpart as a separate step:
  * it is the matmul of packages/core/src/dispatch/matmulOps.ts:32-125 before its epilogue). */

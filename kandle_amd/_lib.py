@@ -88,6 +88,7 @@ SIGNATURES = {
                                    _vp, _i64p, _f, _i64, _i, _vp],
     "kh_rope_table": [_vp, _i64, _vp, _i, _vp],
     "kh_gemm_split_count": [_i64, _i64, _i64, C.POINTER(C.c_int)],
+    "kh_gemm_split_count_for": [_i64, _i64, _i64, _i, C.POINTER(C.c_int)],
     "kh_gemm_splitk_partials": [_vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i, _i],
     "kh_add_rms_norm": [_vp, _i, _i64, _vp, _vp, _vp, _i64, _i64, _f, _i],
 }

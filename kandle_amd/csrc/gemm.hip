@@ -835,16 +835,18 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const TA* __restrict_
 // epilogue.  Per output the large tiles cost the least, but a call takes as many rounds of 256
 // workgroups as its tiles need, so the choice is the smallest ceil(tiles / CUs) * (steps * step + ends).
 // For example 512 x 4096 x 1024 (fp32): 256 tiles of 64 x 128 14.8 us, 128 of 128 x 128 18.9, 512 of
-// 64 x 64 16.7; 1000 x 6144 x 1024: 192 of 128 x 256 33.0 us, 96 of 256 x 256 42, 384 of 128 x 128 40.
+// 64 x 64 16.7; 1000 x 6144 x 1024: 256 of 128 x 192 32.0 us, 192 of 128 x 256 34.2, 96 of 256 x 256 42,
+// 384 of 128 x 128 40; 512 x 6144 x 1024: 256 of 64 x 192 19.8 us, 192 of 128 x 128 21.5.
 struct TileCost {
   int gm, gn;
   float step, ends;
 };
-constexpr int kTiles = 5;
+constexpr int kTiles = 7;
 constexpr TileCost kTileBf16[kTiles] = {
-    {64, 64, .20f, 1.f}, {64, 128, .38f, 1.5f}, {128, 128, .65f, 2.f}, {256, 128, .98f, 3.f}, {256, 256, 1.7f, 5.f}};
+    {64, 64, .20f, 1.f}, {64, 128, .38f, 1.5f}, {128, 128, .65f, 2.f}, {256, 128, .98f, 3.f}, {256, 256, 1.7f, 5.f}, {0, 0, 0.f, 0.f}, {0, 0, 0.f, 0.f}};
 constexpr TileCost kTileF32[kTiles] = {
-    {64, 64, .50f, 1.f}, {64, 128, .71f, 1.5f}, {128, 128, 1.19f, 2.f}, {128, 256, 1.75f, 3.f}, {256, 256, 3.2f, 5.f}};
+    {64, 64, .50f, 1.f}, {64, 128, .71f, 1.5f}, {128, 128, 1.19f, 2.f}, {128, 256, 1.75f, 3.f}, {256, 256, 3.2f, 5.f},
+    {64, 192, .95f, 2.f}, {128, 192, 1.6f, 2.5f}};  // (not whole head rows: no QKNR)
 constexpr int kCUs = 256;
 
 inline float tile_cost(const TileCost& t, int64_t M, int64_t N, int64_t K, int splits) {
@@ -852,11 +854,12 @@ inline float tile_cost(const TileCost& t, int64_t M, int64_t N, int64_t K, int s
   const float steps = (float)((K + 63) / 64) / (float)splits;
   return (float)((blocks + kCUs - 1) / kCUs) * (steps * t.step + t.ends);
 }
-// The tile (from `first` on) of a product split `splits` ways; its cost in *cost if given.
-inline int choose_tile(bool f32, int M, int N, int K, int splits, int first = 0, float* cost = nullptr) {
+// The tile of a product split `splits` ways; its cost in *cost if given.  heads: tiles of whole head rows.
+inline int choose_tile(bool f32, int M, int N, int K, int splits, bool heads = false, float* cost = nullptr) {
+  const int first = heads ? 1 : 0, end = heads || !f32 ? 5 : kTiles;
   int best = first;
   float low = 0.f;
-  for (int i = first; i < kTiles; ++i) {
+  for (int i = first; i < end; ++i) {
     const float c = tile_cost(f32 ? kTileF32[i] : kTileBf16[i], M, N, K, splits);
     if (i == first || c < low) {
       low = c;
@@ -884,17 +887,20 @@ GemmPlan gemm_plan(bool aligned, int64_t lda, int64_t ldb, int M, int N, int K, 
     return p;
   p.mfma = true;
   p.kchunk = K;
-  // The K split (the same for bf16 and fp32 activations, so that kh_gemm_split_count needs no type) is
-  // the cheapest for fp32 ones: a split adds the partials' way through memory (0.35 us a MB) and about
-  // 1 us, and pays where the tiles of whole sums leave CUs idle.  1000 x 1024 x 3072 fp32: 64 x 64 tiles
-  // unsplit 26.8 us, 64 x 128 split in two 19.9; 512 x 1024 x 3072: 23.7 us unsplit, 13.3 split in four.
-  if (K >= 512 && N % 4 == 0) {
+  // The K split: a split adds the partials' way through memory (0.35 us a MB) and about 1 us, and pays
+  // where the tiles of whole sums leave CUs idle.  1000 x 1024 x 3072 fp32: 64 x 64 tiles unsplit 26.8 us,
+  // 64 x 128 split in two 19.9; 512 x 1024 x 3072: 23.7 us unsplit, 13.3 split in four.  bf16 products
+  // (half the work per step) take the same split while 64 x 64 tiles fill less than five eighths of the
+  // CUs, none from there on: 1000 x 1024 x 2048 split in two 10.1 us and 4.7 for the sum, unsplit 9.5;
+  // 1500 x 1024 x 3072 18.5 and 11.4 against 18.6; 2000 x 2560 x 9728 102 and 22 against 125.
+  const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
+  if (K >= 512 && N % 4 == 0 && (a_bytes == 4 || t64 < kCUs * 5 / 8)) {
     float low = 0.f;
     for (int sp = 1; sp <= kMaxSplits; ++sp) {
       const int kchunk = ((K + sp - 1) / sp + 127) / 128 * 128;
       if (sp > 1 && (K + kchunk - 1) / kchunk != sp) continue;
       float c;
-      choose_tile(true, M, N, K, sp, 0, &c);
+      choose_tile(true, M, N, K, sp, false, &c);
       if (sp > 1) c += 1.f + 0.35e-6f * 4.f * (float)sp * (float)M * (float)N;
       if (sp == 1 || c < low) {
         low = c;
@@ -954,6 +960,10 @@ int launch_tile(int tile, const TA* A, int64_t lda, const uint16_t* B, int64_t l
       return go(KH_I(1), KH_I(4), KH_I(4), KH_I(2), KH_I(32), KH_I(4));
     else
       return go(KH_I(2), KH_I(2), KH_I(4), KH_I(2), KH_I(64), KH_I(3));
+  }
+  if constexpr (AF && USE != USE_QKNR) {
+    if (tile == 5) return go(KH_I(1), KH_I(3), KH_I(2), KH_I(2), KH_I(64), KH_I(3));
+    if (tile == 6) return go(KH_I(1), KH_I(3), KH_I(4), KH_I(2), KH_I(64), KH_I(2));
   }
   return go(KH_I(2), KH_I(4), KH_I(4), KH_I(2), KH_I(32), KH_I(AF ? 3 : 4));
 #undef KH_I
@@ -1029,7 +1039,7 @@ int launch_gemm_swiglu(const TA* X, int64_t ldx, const uint16_t* W, int64_t ldw,
 template <typename TA>
 int launch_gemm_qk_norm_rope(const TA* X, int64_t ldx, const uint16_t* W, int64_t ldw, int M, int N, int K,
                              const QknrArgs& qa) {
-  return launch_tile<TA, TA, USE_QKNR>(choose_tile(sizeof(TA) == 4, M, N, K, 1, 1), X, ldx, W, ldw, (TA*)nullptr, 0,
+  return launch_tile<TA, TA, USE_QKNR>(choose_tile(sizeof(TA) == 4, M, N, K, 1, true), X, ldx, W, ldw, (TA*)nullptr, 0,
                                        nullptr, 0, nullptr, M, N, K, 1.f, 0.f, 1, K, nullptr, qa);
 }
 
@@ -1092,8 +1102,16 @@ int kh_gemm_split_count(int64_t m, int64_t n, int64_t k, int* splits) {
   KH_REQUIRE(splits != nullptr, "kh_gemm_split_count: null pointer");
   KH_REQUIRE(m >= 0 && n >= 0 && k >= 0 && m <= INT32_MAX && n <= INT32_MAX && k <= INT32_MAX,
              "kh_gemm_split_count: bad extents");
-  // bf16 weights, contiguous and 16-byte aligned operands (the split does not depend on A's type)
-  const GemmPlan p = gemm_plan(true, k, k, (int)m, (int)n, (int)k, true, 1);
+  return kh_gemm_split_count_for(m, n, k, KH_BF16, splits);
+}
+
+int kh_gemm_split_count_for(int64_t m, int64_t n, int64_t k, int a_dtype, int* splits) {
+  KH_REQUIRE(splits != nullptr, "kh_gemm_split_count_for: null pointer");
+  KH_REQUIRE(m >= 0 && n >= 0 && k >= 0 && m <= INT32_MAX && n <= INT32_MAX && k <= INT32_MAX,
+             "kh_gemm_split_count_for: bad extents");
+  KH_REQUIRE(a_dtype == KH_BF16 || a_dtype == KH_F32, "kh_gemm_split_count_for: unsupported dtype %d", a_dtype);
+  // bf16 weights, contiguous and 16-byte aligned operands
+  const GemmPlan p = gemm_plan(true, k, k, (int)m, (int)n, (int)k, true, 1, a_dtype == KH_F32 ? 4 : 2);
   *splits = p.mfma ? p.splits : 1;
   return KH_OK;
 }
@@ -1107,9 +1125,16 @@ int kh_gemm_splitk_partials(const void* a, int64_t lda, const void* b, int64_t l
   KH_REQUIRE(lda >= k && ldb >= k, "kh_gemm_splitk_partials: leading dimension too small");
   KH_REQUIRE(a_dtype == KH_BF16 || a_dtype == KH_F32, "kh_gemm_splitk_partials: unsupported dtype %d", a_dtype);
   const int ab = a_dtype == KH_F32 ? 4 : 2;
-  const GemmPlan p = gemm_plan(aligned16(a) && aligned16(b), lda, ldb, (int)m, (int)n, (int)k, true, 1, ab);
+  GemmPlan p = gemm_plan(aligned16(a) && aligned16(b), lda, ldb, (int)m, (int)n, (int)k, true, 1, ab);
+  int other = 1;  // the other type's count is taken too: a caller may have asked for it without a type
+  if (kh_gemm_split_count_for(m, n, k, ab == 4 ? KH_BF16 : KH_F32, &other) != KH_OK) return KH_ERR_INVALID;
+  if (splits > 1 && splits == other && splits != p.splits) {
+    p.splits = splits;
+    p.kchunk = (((int)k + splits - 1) / splits + 127) / 128 * 128;
+    p.tile = choose_tile(ab == 4, (int)m, (int)n, (int)k, splits);
+  }
   KH_REQUIRE(p.mfma && p.splits > 1 && p.splits == splits,
-             "kh_gemm_splitk_partials: this product is not split %d ways (kh_gemm_split_count gives the count; "
+             "kh_gemm_splitk_partials: this product is not split %d ways (kh_gemm_split_count_for gives the count; "
              "operands must be 16-byte aligned with k and the leading dimensions multiples of 8)", splits);
   if (a_dtype == KH_F32)
     return launch_tile<float, float, USE_SPLIT>(p.tile, (const float*)a, lda, (const uint16_t*)b, ldb, nullptr, 0,

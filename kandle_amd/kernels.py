@@ -921,10 +921,11 @@ def rope_table(positions: HipTensorHandle, inv_freq: HipTensorHandle,
     return out
 
 
-def gemm_split_count(m: int, n: int, k: int) -> int:
-    """The K split kh_gemm uses for a contiguous bf16 [m, k] x [n, k]^T product (1: none)."""
+def gemm_split_count(m: int, n: int, k: int, dtype: str = BFLOAT16) -> int:
+    """The K split kh_gemm uses for a contiguous [m, k] x [n, k]^T product of bf16 weights and
+    activations of `dtype` (1: none)."""
     out = C.c_int(0)
-    _lib.call("kh_gemm_split_count", int(m), int(n), int(k), C.byref(out))
+    _lib.call("kh_gemm_split_count_for", int(m), int(n), int(k), KH_CODE[dtype], C.byref(out))
     return out.value
 
 
@@ -952,7 +953,7 @@ def linear_add_rms_norm(x, w, residual, norm_weight, eps, output, rows=None) -> 
     for h, nm in ((x, "x"), (w, "w"), (residual, "residual"), (output, "output"), (norm_weight, "norm_weight")):
         if not h.is_contiguous():
             raise ValueError(f"linear_add_rms_norm: {nm} must be contiguous")
-    splits = gemm_split_count(M, N, K)
+    splits = gemm_split_count(M, N, K, x.dtype)
     aligned = all(h.data_ptr() % 16 == 0 for h in (x, w, residual, output, norm_weight))
     if splits > 1 and aligned and N % 8 == 0 and N <= 2048:
         part = HipTensorHandle.create_new((splits, M, N), FLOAT32)

@@ -283,7 +283,7 @@ class Qwen3ForCausalLM:
         # its MFMA tiles (more than 8 rows) without splitting K: only then are the values the same.
         nqkv = (cfg.num_attention_heads + 2 * cfg.num_key_value_heads) * cfg.head_dim
         fuse_qkv = (self.fused_qkv_rope and not one and S > 8
-                    and gemm_split_count(S, nqkv, Hd) == 1)
+                    and gemm_split_count(S, nqkv, Hd, act) == 1)
         # the RoPE angles of these positions, once for every layer's fused projection
         rope_tab = self.ops.find("rope_table")(positions.handle, self.rope.inv_freq.handle) if fuse_qkv else None
         for li, L in enumerate(self.layers):

@@ -664,6 +664,19 @@ static napi_value js_gemmSplitCount(napi_env env, napi_callback_info info) {
   napi_create_int32(env, splits, &out);
   return out;
 }
+/* gemmSplitCountFor(m, n, k, aDtype) -> the same for activations of that type */
+static napi_value js_gemmSplitCountFor(napi_env env, napi_callback_info info) {
+  Args A_, *A = &A_;
+  if (!begin(A, env, info, "gemmSplitCountFor", 4)) return NULL;
+  int64_t m = arg_i64(A, 0), n = arg_i64(A, 1), k = arg_i64(A, 2);
+  int adt = arg_int(A, 3);
+  if (A->bad) return NULL;
+  int splits = 0;
+  if (kh_gemm_split_count_for(m, n, k, adt, &splits) != KH_OK) return done(A, KH_ERR_INVALID);
+  napi_value out;
+  napi_create_int32(env, splits, &out);
+  return out;
+}
 /* gemmSplitkPartials(a, lda, b, ldb, part, m, n, k, splits, aDtype): gemm's split-K stage alone, fp32
    partials [splits][m][n] */
 FN(gemmSplitkPartials, 10)
@@ -708,7 +721,7 @@ static napi_value module_init(napi_env env, napi_value exports) {
       EXPORT(sampleSetPath), EXPORT(philox4x32_10), EXPORT(decodeAttentionBlock), EXPORT(rmsNorm),
       EXPORT(qkNormRope), EXPORT(flashAttention), EXPORT(flashAttentionSplit), EXPORT(flashAttentionMasked), EXPORT(decodeAttention),
       EXPORT(decodeAttentionNoalloc), EXPORT(gemm), EXPORT(gemmEx), EXPORT(gemmSwiglu), EXPORT(gemmQkNormRope), EXPORT(gemmQkNormRopeTable), EXPORT(ropeTable), EXPORT(gemmSplitCount),
-      EXPORT(gemmSplitkPartials), EXPORT(addRmsNorm), EXPORT(gemvFused), EXPORT(gemvSwiglu),
+      EXPORT(gemmSplitCountFor), EXPORT(gemmSplitkPartials), EXPORT(addRmsNorm), EXPORT(gemvFused), EXPORT(gemvSwiglu),
   };
   napi_define_properties(env, exports, sizeof(d) / sizeof(d[0]), d);
   napi_value v;

@@ -890,7 +890,7 @@ function linearAddRmsNorm(x: HipTensorHandle, w: HipTensorHandle, residual: HipT
   if (!(r0 >= 0 && r0 < r1 && r1 <= M)) throw new Error('linear_add_rms_norm: bad row range');
   for (const h of [x, w, residual, out, normWeight])
     if (!h.isContiguous()) throw new Error('linear_add_rms_norm: contiguous operands expected');
-  const splits = addon.gemmSplitCount(M, N, K) as number;
+  const splits = addon.gemmSplitCountFor(M, N, K, x.kh) as number;
   const aligned = [x, w, residual, out, normWeight].every((h) => h.ptr % 16n === 0n);
   const rowOff = BigInt(r0 * N * 4);
   if (splits > 1 && aligned && N % 8 === 0 && N <= 2048) {
@@ -1021,9 +1021,10 @@ export class HipBackend {
     addon.graphDestroy(graph);
   }
 
-  // The K split matmul (kh_gemm) uses for a contiguous bf16 [m, k] x [n, k]^T product (1: none).
-  gemmSplitCount(m: number, n: number, k: number): number {
-    return addon.gemmSplitCount(m, n, k);
+  // The K split matmul (kh_gemm) uses for a contiguous [m, k] x [n, k]^T product of bf16 weights and
+  // activations of `dtype` (1: none).
+  gemmSplitCount(m: number, n: number, k: number, dtype: string = 'bfloat16'): number {
+    return addon.gemmSplitCountFor(m, n, k, DTYPE_CODE[dtype]);
   }
 
   memoryStats(): { [key: string]: number } {

@@ -263,7 +263,7 @@ export class Qwen3ForCausalLM {
     const x = be.createTensorHandle([S, H], 'float32');
     // the fused QKV projection sums over all of K, as matmul does on MFMA tiles (more than 8 rows)
     // when it does not split K
-    const fuseQkv = D === 128 && S > 8 && be.gemmSplitCount(S, nqkv, H) === 1;
+    const fuseQkv = D === 128 && S > 8 && be.gemmSplitCount(S, nqkv, H, act) === 1;
     ops.find('index_select')(this.embed, ids, { dim: 0 }, x);
     let h = ops.find('rms_norm')([x], { normalizedShape: [H], eps, weight: this.layers[0].inNormA, outDtype: act });
     // the RoPE angles of these positions, once for every layer's fused projection

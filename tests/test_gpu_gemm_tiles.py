@@ -1,0 +1,71 @@
+"""The MFMA tile kernel over its tiles and K splits (kh_gemm_ex): edges of rows, columns and k ranges."""
+import numpy as np
+import pytest
+
+import oracle
+from kandle_amd import Tensor, kernels, synthetic as syn
+from kandle_amd import functional as F
+
+pytestmark = pytest.mark.gpu
+
+
+# Rows and columns one short of, on and past tiles of 64 to 256; k of one 16-wide step and less, not a
+# multiple of the 32- and 64-wide stages, and long enough to split; the large ones reach the 128- and
+# 256-wide tiles of each activation type.
+@pytest.mark.parametrize("M,N,K", [
+    (9, 64, 8), (17, 130, 40), (63, 65, 72), (65, 100, 136), (129, 257, 104), (200, 1000, 1016), (257, 300, 2056),
+    (513, 1027, 264), (300, 6144, 520), (700, 6150, 328), (1000, 4100, 200), (2040, 5000, 96)])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_tiles_match_oracle(hip, dtype, M, N, K):
+    """fp32 outputs with the C and bias terms.  fp32 activations are multiplied as a bf16 pair, 2^-16 of
+    each product off at most; the K products are summed in fp32: at most (2^-16 + K 2^-24) sum |a w|
+    (bf16 activations: only the sums), plus 2^-22 of the epilogue's terms."""
+    x = syn.normal(1, (M, K))
+    if dtype == "bfloat16":
+        bits, x = syn.bf16(x)
+        xt = Tensor(bits, dtype=dtype)
+    else:
+        xt = Tensor(x, dtype=dtype)
+    wbits, w = syn.bf16(syn.normal(2, (N, K), 0.05))
+    c, b = syn.normal(3, (M, N)), syn.normal(4, (N,))
+    y = F.dispatch_matmul(xt, Tensor(wbits, dtype="bfloat16"), c=Tensor(c), beta=0.5, alpha=2.0, bias=Tensor(b),
+                          transpose_b=True, out_dtype="float32").numpy()
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    ref = 2.0 * (x64 @ w64.T) + 0.5 * c + b
+    each = (2.0 ** -16 if dtype == "float32" else 0.0) + K * 2.0 ** -24
+    bar = 2.0 * each * (np.abs(x64) @ np.abs(w64).T) + 2.0 ** -22 * (np.abs(ref) + np.abs(c) + np.abs(b) + 1.0)
+    assert np.all(np.abs(y - ref) <= bar), np.max(np.abs(y - ref) - bar)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("M,I,K", [(70, 40, 72), (300, 1504, 136), (512, 3072, 64), (1000, 3080, 40)])
+def test_swiglu_tiles_match_plain_tiles(hip, dtype, M, I, K):
+    """The SwiGLU epilogue, whatever tile runs it, equals silu * mul of the same projection's columns from
+    the plain product, whose sums have the same bits."""
+    def act(seed, shape, std):
+        v = syn.normal(seed, shape, std)
+        return Tensor(syn.bf16(v)[0], dtype=dtype) if dtype == "bfloat16" else Tensor(v, dtype=dtype)
+    x = act(1, (M, K), 1.0)
+    g, u = (syn.bf16(syn.normal(s, (I, K), 0.2))[0] for s in (2, 3))
+    gu = kernels.interleave_gate_up(g, u)
+    got = F.linear_swiglu(x, Tensor(gu, dtype="bfloat16")).numpy()
+    gate, up = (F.linear(x, Tensor(w, dtype="bfloat16")) for w in (g, u))
+    assert kernels.gemm_split_count(M, I, K, dtype) == 1
+    assert np.array_equal(got, F.silu_mul(gate, up).numpy())
+
+
+def test_split_counts_follow_the_activation_type(hip):
+    """kh_gemm_split_count (bf16) and the typed count; partials accept the other type's count."""
+    assert kernels.gemm_split_count(1000, 1024, 3072) == 1
+    n = kernels.gemm_split_count(1000, 1024, 3072, "float32")
+    assert n > 1
+    M, N, K = 1000, 1024, 3072
+    bits, x = syn.bf16(syn.normal(1, (M, K)))
+    wbits, w = syn.bf16(syn.normal(2, (N, K), 0.05))
+    xt, wt = Tensor(bits, dtype="bfloat16"), Tensor(wbits, dtype="bfloat16")
+    part = F.zeros((n, M, N))
+    kernels._lib.call("kh_gemm_splitk_partials", xt.handle.data_ptr(), K, wt.handle.data_ptr(), K, part.handle.data_ptr(),
+                      M, N, K, n, 1)
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    bar = K * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T)
+    assert np.all(np.abs(part.numpy().astype(np.float64).sum(0) - x64 @ w64.T) <= bar)
