@@ -709,9 +709,13 @@ __global__ __launch_bounds__(256) void gemv1_kernel(const void* __restrict__ x, 
   GemvRows<U, PAIR8, EX> g;
   g.init(W, ldw, w_bytes, N, K, nch, (int64_t)blockIdx.x * (blockDim.x >> 6) + w,
          (int64_t)gridDim.x * (blockDim.x >> 6));
+  GemvPrologue<PRO, EX> pro;
+  pro.load(x, nw, K, nch * GV_CHUNK, am);
+  __builtin_amdgcn_sched_barrier(0);
   // The first batch is in flight while the workgroup forms x'.
   g.issue_first();
-  gemv_prologue<PRO, EX>(xs, x, x2, nw, eps, K, nch * GV_CHUNK, am);
+  __builtin_amdgcn_sched_barrier(0);
+  pro.finish(xs, x, x2, nw, eps, K, nch * GV_CHUNK, am);
   g.template run<TO>(xs, C, cin, bias, alpha, beta);
 }
 
