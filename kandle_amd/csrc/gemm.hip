@@ -883,10 +883,10 @@ struct GemmPlan {
 // aligned: both operands start on 16 bytes.  bf16: bf16 weights B with bf16 (a_bytes 2) or fp32
 // (a_bytes 4, split into hi + lo) activations A.
 GemmPlan gemm_plan(bool aligned, int64_t lda, int64_t ldb, int M, int N, int K, bool bf16, int trans_b,
-                   int a_bytes = 2) {
+                   int a_bytes = 2, int min_rows = SK_MAXM + 1) {
   GemmPlan p;
   const int64_t lim = int64_t(1) << 31;
-  if (!(bf16 && trans_b && M > SK_MAXM && K > 0 && K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned &&
+  if (!(bf16 && trans_b && M >= min_rows && K > 0 && K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned &&
         128 * lda * a_bytes < lim && 128 * ldb * 2 < lim))
     return p;
   p.mfma = true;
@@ -983,7 +983,20 @@ int launch_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
   const TO* CI = (const TO*)cin;
   const TO* BI = (const TO*)bias;
   constexpr bool w_bf16 = sizeof(T) == 2;
-  const GemmPlan p = gemm_plan(aligned16(a) && aligned16(b), lda, ldb, M, N, K, w_bf16, trans_b, (int)sizeof(TA));
+  // Two to SK_MAXM rows.  bf16 results come from the tiles, which read the weights once whatever the rows,
+  // where the skinny kernel re-reads its fp32 rows from LDS for every four weight rows: 5 x 1024 x 1024
+  // 17.9 -> 8.3 us, 2 x 6144 x 2560 28.5 -> 11.3, 8 x 151936 x 1024 541 -> 58; two short rows against few
+  // columns stay (2 x 1024 rows against a few thousand columns: 11.0 there, 12.3 on tiles, one call in turn).  fp32 results keep the
+  // skinny kernel's 64-way sums (error against 64 bits 7e-8 at K = 1024, the tiles' 8e-8) as long as its rows
+  // fit LDS; beyond, the generic kernel's one sum over K (1e-6 at K = 9728) was both slower and less
+  // exact: bf16 rows take the tiles there (8 x 2560 x 9728 1529 -> 13.9 us, error 2.5e-7), fp32 rows the
+  // one-row kernel row by row (1542 -> 141 us, 2.3e-7; its exact products, which the tiles' split of
+  // fp32 rows into two bf16 would not keep).
+  const bool skinny_fits = M <= SK_MAXM && (size_t)M * K * sizeof(float) <= 64 * 1024;
+  const bool few_tiles = sizeof(TO) == 2 && (M > 2 || K > 1024 || N > 4096);
+  const int min_rows = sizeof(TA) == 2 && (few_tiles || !skinny_fits) ? 2 : SK_MAXM + 1;
+  const GemmPlan p =
+      gemm_plan(aligned16(a) && aligned16(b), lda, ldb, M, N, K, w_bf16, trans_b, (int)sizeof(TA), min_rows);
   if constexpr (w_bf16) {
     if (p.mfma) {
       if (p.splits > 1) {
@@ -1011,8 +1024,19 @@ int launch_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
         return KH_OK;
       }
     }
+    if constexpr (std::is_same<TA, float>::value) {
+      if (trans_b && M > 1 && M <= SK_MAXM && !skinny_fits) {
+        int m = 0;
+        while (m < M && launch_gemv1<PRO_NONE, TO, true>(A + m * lda, nullptr, nullptr, 0.f, (const uint16_t*)B, ldb,
+                                                         C + m * ldc, CI ? CI + m * ldcin : nullptr, BI, N, K, alpha, beta))
+          ++m;
+        KH_CHECK_LAUNCH();
+        if (m == M) return KH_OK;
+        KH_REQUIRE(m == 0, "kh_gemm: row %d of %d was refused", m, M);
+      }
+    }
   }
-  if (trans_b && M <= SK_MAXM && (size_t)M * K * sizeof(float) <= 64 * 1024 && aligned16(b)) {
+  if (trans_b && skinny_fits && aligned16(b)) {
     const int waves_needed = (N + SK_ROWS_PER_WAVE - 1) / SK_ROWS_PER_WAVE;
     int grid = (waves_needed + 3) / 4;
     if (grid > 4096) grid = 4096;
