@@ -986,7 +986,7 @@ int launch_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
   // Two to SK_MAXM rows.  bf16 results come from the tiles, which read the weights once whatever the rows,
   // where the skinny kernel re-reads its fp32 rows from LDS for every four weight rows: 5 x 1024 x 1024
   // 17.9 -> 8.3 us, 2 x 6144 x 2560 28.5 -> 11.3, 8 x 151936 x 1024 541 -> 58; two short rows against few
-  // columns stay (2 x 1024 rows against a few thousand columns: 11.0 there, 12.3 on tiles, one call in turn).  fp32 results keep the
+  // columns stay (2 x 4096 x 1024: 11.0 there, 12.3 on tiles).  fp32 results keep the
   // skinny kernel's 64-way sums (error against 64 bits 7e-8 at K = 1024, the tiles' 8e-8) as long as its rows
   // fit LDS; beyond, the generic kernel's one sum over K (1e-6 at K = 9728) was both slower and less
   // exact: bf16 rows take the tiles there (8 x 2560 x 9728 1529 -> 13.9 us, error 2.5e-7), fp32 rows the
