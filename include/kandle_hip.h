@@ -435,7 +435,7 @@ int kh_rope_table(const int32_t* positions, int64_t n, const float* inv_freq, in
 
 /* The split count kh_gemm uses for a bf16 [m, k] x [n, k]^T product with contiguous, 16-byte aligned
  * operands (1: not split).  A caller that splits the same product with kh_gemm_splitk_partials and
- * adds the partials in split order reproduces kh_gemm bit for bit. */
+ * adds the partials in split order reproduces kh_gemm with fp32 results bit for bit. */
 int kh_gemm_split_count(int64_t m, int64_t n, int64_t k, int* splits);
 
 /* The same for an A of type a_dtype (KH_BF16 or KH_F32) and bf16 weights (kh_gemm_ex). */

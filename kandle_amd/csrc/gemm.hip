@@ -312,6 +312,12 @@ __device__ __forceinline__ void gemm_wave_store(const f32x16 (&acc)[AN][AM], cha
 //   bf16 1000 x 6144 x 1024  30.9 -> 20.1 us     fp32 1000 x 6144 x 1024  55.1 -> 33.0 us
 //   bf16 2000 x 19456 x 2560  339 ->  240 us     fp32 2000 x 19456 x 2560  600 -> 405 us
 // Rows past M or N repeat the last one and are never stored; columns past the k range read as zero.
+//
+// PARTS (bf16 activations, long fp32 sums of few tiles): each of a stage's four 16-wide steps has an
+// accumulator of its own, added at the end: the chains of fp32 additions are those of a product split in
+// four.  A chain of n steps is about 2^-24 sqrt(n / 6) of the result off: 640 x 1024 x 2048 1.3e-7 against
+// 64 bits (one accumulator 2.7e-7), 256 x 2560 x 9728 3.0e-7 (6.3e-7), 128 x 4096 x 1024 split in two
+// 8e-8 (1.3e-7).  The additions at the end take 0.2-0.3 us (640 x 1024 x 2048 8.8 -> 9.1).
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // 64 lanes x 16 bytes from rsrc at byte voff (per lane) + soff to LDS byte address lds + 16 lane.
@@ -367,7 +373,7 @@ __device__ __forceinline__ int lds_swz(int row) {
 }
 
 template <typename TO, int AM, int AN, int WM, int WN, int KS, int NST, bool SPLIT, bool SWIGLU, bool QKNR,
-          typename TA>
+          bool PARTS, typename TA>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(
     const TA* __restrict__ A, int64_t lda, const uint16_t* __restrict__ B, int64_t ldb, TO* C, int64_t ldc,
     const TO* cin, int64_t ldcin, const TO* __restrict__ bias, int M, int N, int K, float alpha, float beta,
@@ -420,14 +426,18 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(
                     base + T::ABYTES + (i - T::LA) * NW * 1024);
   };
 
-  f32x16 acc[AN][AM];
+  constexpr int KC = KS / 16, ALL = KC * AN;  // 16-wide steps of a stage, and places between its products
+  constexpr int SETS = PARTS ? KC : 1;
+  f32x16 sums[SETS][AN][AM];
 #pragma unroll
-  for (int a = 0; a < AN; ++a)
+  for (int s = 0; s < SETS; ++s)
 #pragma unroll
-    for (int b = 0; b < AM; ++b)
+    for (int a = 0; a < AN; ++a)
 #pragma unroll
-      for (int j = 0; j < 16; ++j) acc[a][b][j] = 0.f;
-
+      for (int b = 0; b < AM; ++b)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) sums[s][a][b][j] = 0.f;
+  auto& acc = sums[0];
   // Fragments of one 16-wide k step: B rows, and A rows as stored (fp32: two 16-byte halves) until
   // split_a makes them bf16 (fp32: hi and lo).
   constexpr int AW = AF ? 2 : 1;
@@ -466,26 +476,28 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(
       }
     }
   };
-  auto multiply = [&](const Frag& f, int pl, auto&& between) {
+  // kc: the step of its stage that f holds
+  auto multiply = [&](const Frag& f, int kc, int pl, auto&& between) {
+    auto& to = sums[PARTS ? kc : 0];
 #pragma unroll
     for (int a = 0; a < AN; ++a) {
 #pragma unroll
       for (int b = 0; b < AM; ++b)
-        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(f.b[a]), as_bf16x8(f.a[b][pl]), acc[a][b], 0, 0, 0);
+        to[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(f.b[a]), as_bf16x8(f.a[b][pl]), to[a][b], 0, 0, 0);
       between(a);
     }
   };
   auto nothing = [](int) {};
-  // One 16-wide step: read the next step's fragments, multiply this one's; with fp32 activations the
+  // One 16-wide step: read the next step's (kc) fragments, multiply this one's (kc - 1, or the last); with fp32 activations the
   // next fragments are split in the shadow of the second plane's products.
   auto step = [&](Frag& cur, Frag& nxt, int buf, int kc, auto&& between) {
     read_frag(nxt, buf, kc);
     __builtin_amdgcn_sched_barrier(0);
-    multiply(cur, 0, between);
+    multiply(cur, (kc + KC - 1) % KC, 0, between);
     if constexpr (AF) {
       __builtin_amdgcn_sched_barrier(0);
       split_a(nxt);
-      multiply(cur, AW - 1, nothing);
+      multiply(cur, (kc + KC - 1) % KC, AW - 1, nothing);
 #pragma unroll
       for (int i = 0; i < AN * AM; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                            // one MFMA
@@ -501,7 +513,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(
   // the copies of the stage NST later.  Those are issued one by one between the products of the steps
   // that follow, up to the next stage's barrier: issued together they keep the matrix cores waiting
   // for the address unit (64 bytes per cycle).
-  constexpr int KC = KS / 16, ALL = KC * AN;
   Frag fr[2];
   if (nk > 0) {
 #pragma unroll
@@ -554,8 +565,18 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(
 #pragma unroll
       for (int kc = 0; kc + 1 < KC; ++kc) step(fr[kc & 1], fr[(kc + 1) & 1], buf, kc + 1, nothing);
     }
-    multiply(fr[1], 0, nothing);
-    if constexpr (AF) multiply(fr[1], AW - 1, nothing);
+    multiply(fr[1], KC - 1, 0, nothing);
+    if constexpr (AF) multiply(fr[1], KC - 1, AW - 1, nothing);
+    if constexpr (PARTS) {
+      static_assert(!AF && KC == 4, "four steps per stage");
+#pragma unroll
+      for (int a = 0; a < AN; ++a)
+#pragma unroll
+        for (int b = 0; b < AM; ++b)
+#pragma unroll
+          for (int j = 0; j < 16; ++j)
+            acc[a][b][j] = (acc[a][b][j] + sums[1][a][b][j]) + (sums[SETS - 2][a][b][j] + sums[SETS - 1][a][b][j]);
+    }
   }
   __syncthreads();  // the tile is stored by way of the loop's LDS
   if constexpr (QKNR) {
@@ -917,18 +938,29 @@ GemmPlan gemm_plan(bool aligned, int64_t lda, int64_t ldb, int M, int N, int K, 
   return p;
 }
 
+// Long fp32 sums of bf16 products whose 64 x 64 tiles leave CUs idle, split in fewer ways than would put
+// two such tiles on every CU, are taken in PARTS: the wider split can cost more than it gains (the
+// partials' way through memory), but its shorter chains are worth keeping.
+inline bool sums_in_parts(int64_t M, int64_t N, int K, int splits) {
+  const int64_t t64 = ((M + 63) / 64) * ((N + 63) / 64);
+  if (!(K >= 1024 && N % 4 == 0 && t64 < kCUs)) return false;
+  const int64_t want = 2 * kCUs / t64 > kMaxSplits ? kMaxSplits : 2 * kCUs / t64;
+  const int64_t kchunk = ((K + want - 1) / want + 127) / 128 * 128;
+  return splits < (K + kchunk - 1) / kchunk;
+}
+
 enum TileUse { USE_PLAIN, USE_SPLIT, USE_SWIGLU, USE_QKNR };
 
 // One launch of the tile kernel: AM x AN blocks of 32 x 32 outputs per wave, WM x WN waves, NST stages
 // of KS columns in LDS.
-template <typename TO, typename TA, TileUse USE, int AM, int AN, int WM, int WN, int KS, int NST>
+template <typename TO, typename TA, TileUse USE, bool PARTS, int AM, int AN, int WM, int WN, int KS, int NST>
 int go_tile(const TA* A, int64_t lda, const uint16_t* B, int64_t ldb, TO* C, int64_t ldc, const TO* CI, int64_t ldcin,
             const TO* BI, int M, int N, int K, float alpha, float beta, int splits, int kchunk, float* part,
             const QknrArgs& qa) {
   using T = DmaTile<TA, AM, AN, WM, WN, KS>;
   const int64_t blocks = (int64_t)((M + T::GM - 1) / T::GM) * ((N + T::GN - 1) / T::GN) * splits;
   KH_REQUIRE(blocks <= INT32_MAX, "kh_gemm: grid too large");
-  gemm_tile_kernel<TO, AM, AN, WM, WN, KS, NST, USE == USE_SPLIT, USE == USE_SWIGLU, USE == USE_QKNR, TA>
+  gemm_tile_kernel<TO, AM, AN, WM, WN, KS, NST, USE == USE_SPLIT, USE == USE_SWIGLU, USE == USE_QKNR, PARTS, TA>
       <<<(int)blocks, 64 * WM * WN, 0, stream()>>>(A, lda, B, ldb, C, ldc, CI, ldcin, BI, M, N, K, alpha, beta, splits,
                                                    kchunk, part, qa);
   KH_CHECK_LAUNCH();
@@ -937,16 +969,24 @@ int go_tile(const TA* A, int64_t lda, const uint16_t* B, int64_t ldb, TO* C, int
 
 // The tile kernel with tile `tile` of kTileBf16 / kTileF32.  k-steps of 64 columns; of 32 where two or
 // three stages of 64 do not fit the CU's 160 KiB of LDS.  64 x 128 fp32 tiles run four waves of 32 x 64
-// (each A fragment split by two waves, not four: 16.6 -> 14.8 us at 512 x 4096 x 1024).
+// (each A fragment split by two waves, not four: 16.6 -> 14.8 us at 512 x 4096 x 1024).  f32_result: of
+// USE_SPLIT, whether the partials end as fp32.
 template <typename TO, typename TA, TileUse USE>
 int launch_tile(int tile, const TA* A, int64_t lda, const uint16_t* B, int64_t ldb, TO* C, int64_t ldc, const TO* CI,
                 int64_t ldcin, const TO* BI, int M, int N, int K, float alpha, float beta, int splits, int kchunk,
-                float* part, const QknrArgs& qa = QknrArgs{}) {
+                float* part, const QknrArgs& qa = QknrArgs{}, bool f32_result = true) {
   constexpr bool AF = std::is_same<TA, float>::value;
+  constexpr bool F32SUM = !AF && sizeof(TO) == 4 && (USE == USE_PLAIN || USE == USE_SPLIT);
+  const bool parts = F32SUM && f32_result && sums_in_parts(M, N, K, splits);
   auto go = [&](auto am, auto an, auto wm, auto wn, auto ks, auto nst) {
-    return go_tile<TO, TA, USE, decltype(am)::value, decltype(an)::value, decltype(wm)::value, decltype(wn)::value,
-                   decltype(ks)::value, decltype(nst)::value>(A, lda, B, ldb, C, ldc, CI, ldcin, BI, M, N, K, alpha,
-                                                              beta, splits, kchunk, part, qa);
+    constexpr int AM = decltype(am)::value, AN = decltype(an)::value, WM = decltype(wm)::value, WN = decltype(wn)::value,
+                  KS = decltype(ks)::value, NST = decltype(nst)::value;
+    if constexpr (F32SUM && AM * AN <= 2)  // the tiles that sums_in_parts' products take
+      if (parts)
+        return go_tile<TO, TA, USE, true, AM, AN, WM, WN, KS, NST>(A, lda, B, ldb, C, ldc, CI, ldcin, BI, M, N, K,
+                                                                   alpha, beta, splits, kchunk, part, qa);
+    return go_tile<TO, TA, USE, false, AM, AN, WM, WN, KS, NST>(A, lda, B, ldb, C, ldc, CI, ldcin, BI, M, N, K, alpha,
+                                                                beta, splits, kchunk, part, qa);
   };
   auto c = [](auto v) { return v; };
 #define KH_I(v) c(std::integral_constant<int, (v)>{})
@@ -1003,7 +1043,8 @@ int launch_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
         float* part = (float*)scratch_alloc((size_t)p.splits * M * N * sizeof(float));
         if (part != nullptr) {
           const int rc = launch_tile<float, TA, USE_SPLIT>(p.tile, A, lda, (const uint16_t*)B, ldb, nullptr, 0, nullptr,
-                                                           0, nullptr, M, N, K, alpha, beta, p.splits, p.kchunk, part);
+                                                           0, nullptr, M, N, K, alpha, beta, p.splits, p.kchunk, part,
+                                                           QknrArgs{}, sizeof(TO) == 4);
           if (rc == KH_OK)
             gemm_splitk_reduce_kernel<TO><<<(int)(((int64_t)M * N / 4 + 255) / 256), 256, 0, stream()>>>(
                 part, p.splits, C, ldc, CI, ldcin, BI, M, N, alpha, beta);

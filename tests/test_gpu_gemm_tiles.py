@@ -69,3 +69,20 @@ def test_split_counts_follow_the_activation_type(hip):
     x64, w64 = x.astype(np.float64), w.astype(np.float64)
     bar = K * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T)
     assert np.all(np.abs(part.numpy().astype(np.float64).sum(0) - x64 @ w64.T) <= bar)
+
+
+@pytest.mark.parametrize("M,N,K", [(640, 1024, 2048), (128, 4096, 1024), (960, 1024, 3072), (200, 2560, 4096),
+                                   (100, 6144, 2560), (9, 2560, 4096), (256, 2560, 9728), (900, 1004, 1024)])
+def test_bf16_products_sum_fp32_results_in_short_chains(hip, M, N, K):
+    """fp32 results of bf16 products of few tiles.  A chain of n 16-wide steps of like products has a
+    rounding error of about 2^-24 sqrt(n / 6) of the result (step i adds half a unit, uniformly, of a sum of
+    i of the n steps); n = K / 16 split over the workgroups that put two 64 x 64 tiles on a CU, at most
+    eight, is the longest chain.  One chain of twice that is sqrt(2) off the bar, and the whole K more."""
+    parts = min(8, 512 // (-(-M // 64) * -(-N // 64)))
+    bits, x = syn.bf16(syn.normal(1, (M, K)))
+    wbits, w = syn.bf16(syn.normal(2, (N, K), 0.02))
+    y = F.dispatch_matmul(Tensor(bits, dtype="bfloat16"), Tensor(wbits, dtype="bfloat16"), transpose_b=True,
+                          out_dtype="float32").numpy().astype(np.float64)
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    err = np.linalg.norm(y - ref) / np.linalg.norm(ref)
+    assert err <= 1.1 * 2.0 ** -24 * np.sqrt(K / (16.0 * max(2, parts) * 6.0)), err
