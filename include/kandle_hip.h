@@ -433,9 +433,10 @@ int kh_gemm_qk_norm_rope_table(const void* x, int64_t ldx, const void* w_qkv, in
  * QKV projection (kh_gemm_qk_norm_rope_table). */
 int kh_rope_table(const int32_t* positions, int64_t n, const float* inv_freq, int half, float* out);
 
-/* The split count kh_gemm uses for a bf16 [m, k] x [n, k]^T product with contiguous, 16-byte aligned
- * operands (1: not split).  A caller that splits the same product with kh_gemm_splitk_partials and
- * adds the partials in split order reproduces kh_gemm with fp32 results bit for bit. */
+/* The split count kh_gemm uses for a bf16 [m, k] x [n, k]^T product with fp32 results and contiguous,
+ * 16-byte aligned operands (1: not split).  A caller that splits the same product with
+ * kh_gemm_splitk_partials and adds the partials in split order reproduces kh_gemm bit for bit.  (bf16
+ * results of more than 8 rows are split alike.) */
 int kh_gemm_split_count(int64_t m, int64_t n, int64_t k, int* splits);
 
 /* The same for an A of type a_dtype (KH_BF16 or KH_F32) and bf16 weights (kh_gemm_ex). */

@@ -895,6 +895,23 @@ inline int choose_tile(bool f32, int M, int N, int K, int splits, bool heads = f
   return best;
 }
 
+// The skinny kernel's fp32 rows fit its LDS.
+inline bool fits_skinny(int64_t M, int64_t K) { return M <= SK_MAXM && M * K * (int64_t)sizeof(float) <= 64 * 1024; }
+
+// Two to SK_MAXM rows.  bf16 results come from the tiles, which read the weights once whatever the rows,
+// where the skinny kernel re-reads its fp32 rows from LDS for every four weight rows: 5 x 1024 x 1024
+// 17.9 -> 8.3 us, 2 x 6144 x 2560 28.5 -> 11.3, 8 x 151936 x 1024 541 -> 58; two short rows against few
+// columns stay (2 x 4096 x 1024: 11.0 there, 12.3 on tiles).  fp32 results keep the
+// skinny kernel's 64-way sums (error against 64 bits 7e-8 at K = 1024, the tiles' 8e-8) as long as its rows
+// fit LDS; beyond, the generic kernel's one sum over K (1e-6 at K = 9728) was both slower and less
+// exact: bf16 rows take the tiles there (8 x 2560 x 9728 1529 -> 13.9 us, error 2.5e-7), fp32 rows the
+// one-row kernel row by row (1542 -> 141 us, 2.3e-7; its exact products, which the tiles' split of
+// fp32 rows into two bf16 would not keep).
+inline int tile_min_rows(int a_bytes, int out_bytes, int M, int N, int K) {
+  const bool few_tiles = out_bytes == 2 && (M > 2 || K > 1024 || N > 4096);
+  return a_bytes == 2 && (few_tiles || !fits_skinny(M, K)) ? 2 : SK_MAXM + 1;
+}
+
 // Launch plan of the MFMA tile kernel for a bf16 (or fp32) [M, K] x bf16 [N, K]^T product.
 struct GemmPlan {
   bool mfma = false;  // the MFMA tile kernel applies (else the skinny or generic kernel)
@@ -904,7 +921,7 @@ struct GemmPlan {
 // aligned: both operands start on 16 bytes.  bf16: bf16 weights B with bf16 (a_bytes 2) or fp32
 // (a_bytes 4, split into hi + lo) activations A.
 GemmPlan gemm_plan(bool aligned, int64_t lda, int64_t ldb, int M, int N, int K, bool bf16, int trans_b,
-                   int a_bytes = 2, int min_rows = SK_MAXM + 1) {
+                   int a_bytes, int min_rows) {
   GemmPlan p;
   const int64_t lim = int64_t(1) << 31;
   if (!(bf16 && trans_b && M >= min_rows && K > 0 && K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned &&
@@ -1023,18 +1040,8 @@ int launch_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
   const TO* CI = (const TO*)cin;
   const TO* BI = (const TO*)bias;
   constexpr bool w_bf16 = sizeof(T) == 2;
-  // Two to SK_MAXM rows.  bf16 results come from the tiles, which read the weights once whatever the rows,
-  // where the skinny kernel re-reads its fp32 rows from LDS for every four weight rows: 5 x 1024 x 1024
-  // 17.9 -> 8.3 us, 2 x 6144 x 2560 28.5 -> 11.3, 8 x 151936 x 1024 541 -> 58; two short rows against few
-  // columns stay (2 x 4096 x 1024: 11.0 there, 12.3 on tiles).  fp32 results keep the
-  // skinny kernel's 64-way sums (error against 64 bits 7e-8 at K = 1024, the tiles' 8e-8) as long as its rows
-  // fit LDS; beyond, the generic kernel's one sum over K (1e-6 at K = 9728) was both slower and less
-  // exact: bf16 rows take the tiles there (8 x 2560 x 9728 1529 -> 13.9 us, error 2.5e-7), fp32 rows the
-  // one-row kernel row by row (1542 -> 141 us, 2.3e-7; its exact products, which the tiles' split of
-  // fp32 rows into two bf16 would not keep).
-  const bool skinny_fits = M <= SK_MAXM && (size_t)M * K * sizeof(float) <= 64 * 1024;
-  const bool few_tiles = sizeof(TO) == 2 && (M > 2 || K > 1024 || N > 4096);
-  const int min_rows = sizeof(TA) == 2 && (few_tiles || !skinny_fits) ? 2 : SK_MAXM + 1;
+  const bool skinny_fits = fits_skinny(M, K);
+  const int min_rows = tile_min_rows((int)sizeof(TA), (int)sizeof(TO), M, N, K);
   const GemmPlan p =
       gemm_plan(aligned16(a) && aligned16(b), lda, ldb, M, N, K, w_bf16, trans_b, (int)sizeof(TA), min_rows);
   if constexpr (w_bf16) {
@@ -1179,8 +1186,10 @@ int kh_gemm_split_count_for(int64_t m, int64_t n, int64_t k, int a_dtype, int* s
   KH_REQUIRE(m >= 0 && n >= 0 && k >= 0 && m <= INT32_MAX && n <= INT32_MAX && k <= INT32_MAX,
              "kh_gemm_split_count_for: bad extents");
   KH_REQUIRE(a_dtype == KH_BF16 || a_dtype == KH_F32, "kh_gemm_split_count_for: unsupported dtype %d", a_dtype);
-  // bf16 weights, contiguous and 16-byte aligned operands
-  const GemmPlan p = gemm_plan(true, k, k, (int)m, (int)n, (int)k, true, 1, a_dtype == KH_F32 ? 4 : 2);
+  // bf16 weights, fp32 results, contiguous and 16-byte aligned operands
+  const int ab = a_dtype == KH_F32 ? 4 : 2;
+  const GemmPlan p = gemm_plan(true, k, k, (int)m, (int)n, (int)k, true, 1, ab,
+                               tile_min_rows(ab, 4, (int)m, (int)n, (int)k));
   *splits = p.mfma ? p.splits : 1;
   return KH_OK;
 }
@@ -1194,7 +1203,8 @@ int kh_gemm_splitk_partials(const void* a, int64_t lda, const void* b, int64_t l
   KH_REQUIRE(lda >= k && ldb >= k, "kh_gemm_splitk_partials: leading dimension too small");
   KH_REQUIRE(a_dtype == KH_BF16 || a_dtype == KH_F32, "kh_gemm_splitk_partials: unsupported dtype %d", a_dtype);
   const int ab = a_dtype == KH_F32 ? 4 : 2;
-  GemmPlan p = gemm_plan(aligned16(a) && aligned16(b), lda, ldb, (int)m, (int)n, (int)k, true, 1, ab);
+  GemmPlan p = gemm_plan(aligned16(a) && aligned16(b), lda, ldb, (int)m, (int)n, (int)k, true, 1, ab,
+                         tile_min_rows(ab, 4, (int)m, (int)n, (int)k));
   int other = 1;  // the other type's count is taken too: a caller may have asked for it without a type
   if (kh_gemm_split_count_for(m, n, k, ab == 4 ? KH_BF16 : KH_F32, &other) != KH_OK) return KH_ERR_INVALID;
   if (splits > 1 && splits == other && splits != p.splits) {

@@ -41,3 +41,28 @@ def test_few_rows_match_float64(hip, act, out, M, N, K):
     if out == "bfloat16":
         bar = bar + 2.0 ** -8 * (np.abs(ref) + bar)
     assert np.all(np.abs(y - ref) <= bar), np.max(np.abs(y - ref) - bar)
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 1024, 3072), (5, 256, 4104), (2, 64, 8200), (8, 1024, 1024), (9, 1024, 3072)])
+def test_split_count_of_few_rows(hip, M, N, K):
+    """The count is kh_gemm's with fp32 results also where two to eight bf16 rows are too long for the skinny
+    kernel's LDS (M K > 16384) and take the tiles: kh_gemm's result is its partials added in split order, bit
+    for bit.  fp32 rows are not split there."""
+    from kandle_amd import kernels
+    bits, _ = syn.bf16(syn.normal(1, (M, K)))
+    wbits, _ = syn.bf16(syn.normal(2, (N, K), 0.05))
+    xt, wt = Tensor(bits, dtype="bfloat16"), Tensor(wbits, dtype="bfloat16")
+    n = kernels.gemm_split_count(M, N, K, "bfloat16")
+    if M <= 8:
+        assert (n > 1) == (M * K > 16384)
+        assert kernels.gemm_split_count(M, N, K, "float32") == 1
+    if n == 1:
+        return
+    y = F.dispatch_matmul(xt, wt, transpose_b=True, out_dtype="float32").numpy()
+    part = F.zeros((n, M, N))
+    kernels._lib.call("kh_gemm_splitk_partials", xt.handle.data_ptr(), K, wt.handle.data_ptr(), K,
+                      part.handle.data_ptr(), M, N, K, n, 1)
+    total = np.zeros((M, N), np.float32)
+    for p in part.numpy():
+        total += p
+    assert np.array_equal(total, y)
