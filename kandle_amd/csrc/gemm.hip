@@ -916,7 +916,19 @@ inline int tile_min_rows(int a_bytes, int out_bytes, int M, int N, int K) {
 struct GemmPlan {
   bool mfma = false;  // the MFMA tile kernel applies (else the skinny or generic kernel)
   int tile = 0, splits = 1, kchunk = 0;
+  bool parts = false;  // fp32 results of bf16 products are summed in PARTS
 };
+
+// Long fp32 sums of bf16 products whose 64 x 64 tiles leave CUs idle, split in fewer ways than would put
+// two such tiles on every CU, are taken in PARTS: the wider split can cost more than it gains (the
+// partials' way through memory), but its shorter chains are worth keeping.
+inline bool narrow_split(int64_t M, int64_t N, int K, int splits) {
+  const int64_t t64 = ((M + 63) / 64) * ((N + 63) / 64);
+  if (!(K >= 1024 && N % 4 == 0 && t64 < kCUs)) return false;
+  const int64_t want = 2 * kCUs / t64 > kMaxSplits ? kMaxSplits : 2 * kCUs / t64;
+  const int64_t kchunk = ((K + want - 1) / want + 127) / 128 * 128;
+  return splits < (K + kchunk - 1) / kchunk;
+}
 
 // aligned: both operands start on 16 bytes.  bf16: bf16 weights B with bf16 (a_bytes 2) or fp32
 // (a_bytes 4, split into hi + lo) activations A.
@@ -935,6 +947,10 @@ GemmPlan gemm_plan(bool aligned, int64_t lda, int64_t ldb, int M, int N, int K, 
   // (half the work per step) take the same split while 64 x 64 tiles fill less than five eighths of the
   // CUs, none from there on: 1000 x 1024 x 2048 split in two 10.1 us and 4.7 for the sum, unsplit 9.5;
   // 1500 x 1024 x 3072 18.5 and 11.4 against 18.6; 2000 x 2560 x 9728 102 and 22 against 125.
+  // Sums shorter than 1024 are split only while the tiles are few for their length: 512 x 1024 x 640 (128
+  // tiles) bf16 split in two 8.2 us, whole 4.9, fp32 10.4 and 8.1; 128 x 1024 x 640 (32) bf16 6.6 and 4.7, fp32
+  // 7.5 and 7.7; 300 x 1024 x 1000 (80) fp32 10.2 and 10.9.  (fp32 results of bf16 products keep the short
+  // chains: 512 x 512 x 512 is 1.2e-7 off 64 bits in one chain, 6.3e-8 in PARTS.)
   const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
   if (K >= 512 && N % 4 == 0 && (a_bytes == 4 || t64 < kCUs * 5 / 8)) {
     float low = 0.f;
@@ -951,19 +967,15 @@ GemmPlan gemm_plan(bool aligned, int64_t lda, int64_t ldb, int M, int N, int K, 
       }
     }
   }
+  if (p.splits > 1 && K < 1024 && t64 * (a_bytes == 4 ? 12 : 20) >= K) {
+    p.splits = 1;
+    p.kchunk = K;
+    p.parts = a_bytes == 2;
+  } else {
+    p.parts = a_bytes == 2 && narrow_split(M, N, K, p.splits);
+  }
   p.tile = choose_tile(a_bytes == 4, M, N, K, p.splits);
   return p;
-}
-
-// Long fp32 sums of bf16 products whose 64 x 64 tiles leave CUs idle, split in fewer ways than would put
-// two such tiles on every CU, are taken in PARTS: the wider split can cost more than it gains (the
-// partials' way through memory), but its shorter chains are worth keeping.
-inline bool sums_in_parts(int64_t M, int64_t N, int K, int splits) {
-  const int64_t t64 = ((M + 63) / 64) * ((N + 63) / 64);
-  if (!(K >= 1024 && N % 4 == 0 && t64 < kCUs)) return false;
-  const int64_t want = 2 * kCUs / t64 > kMaxSplits ? kMaxSplits : 2 * kCUs / t64;
-  const int64_t kchunk = ((K + want - 1) / want + 127) / 128 * 128;
-  return splits < (K + kchunk - 1) / kchunk;
 }
 
 enum TileUse { USE_PLAIN, USE_SPLIT, USE_SWIGLU, USE_QKNR };
@@ -986,19 +998,17 @@ int go_tile(const TA* A, int64_t lda, const uint16_t* B, int64_t ldb, TO* C, int
 
 // The tile kernel with tile `tile` of kTileBf16 / kTileF32.  k-steps of 64 columns; of 32 where two or
 // three stages of 64 do not fit the CU's 160 KiB of LDS.  64 x 128 fp32 tiles run four waves of 32 x 64
-// (each A fragment split by two waves, not four: 16.6 -> 14.8 us at 512 x 4096 x 1024).  f32_result: of
-// USE_SPLIT, whether the partials end as fp32.
+// (each A fragment split by two waves, not four: 16.6 -> 14.8 us at 512 x 4096 x 1024).
 template <typename TO, typename TA, TileUse USE>
 int launch_tile(int tile, const TA* A, int64_t lda, const uint16_t* B, int64_t ldb, TO* C, int64_t ldc, const TO* CI,
                 int64_t ldcin, const TO* BI, int M, int N, int K, float alpha, float beta, int splits, int kchunk,
-                float* part, const QknrArgs& qa = QknrArgs{}, bool f32_result = true) {
+                float* part, const QknrArgs& qa = QknrArgs{}, bool parts = false) {
   constexpr bool AF = std::is_same<TA, float>::value;
   constexpr bool F32SUM = !AF && sizeof(TO) == 4 && (USE == USE_PLAIN || USE == USE_SPLIT);
-  const bool parts = F32SUM && f32_result && sums_in_parts(M, N, K, splits);
   auto go = [&](auto am, auto an, auto wm, auto wn, auto ks, auto nst) {
     constexpr int AM = decltype(am)::value, AN = decltype(an)::value, WM = decltype(wm)::value, WN = decltype(wn)::value,
                   KS = decltype(ks)::value, NST = decltype(nst)::value;
-    if constexpr (F32SUM && AM * AN <= 2)  // the tiles that sums_in_parts' products take
+    if constexpr (F32SUM && AM * AN <= 2)  // the tiles that a plan with parts takes
       if (parts)
         return go_tile<TO, TA, USE, true, AM, AN, WM, WN, KS, NST>(A, lda, B, ldb, C, ldc, CI, ldcin, BI, M, N, K,
                                                                    alpha, beta, splits, kchunk, part, qa);
@@ -1051,7 +1061,7 @@ int launch_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
         if (part != nullptr) {
           const int rc = launch_tile<float, TA, USE_SPLIT>(p.tile, A, lda, (const uint16_t*)B, ldb, nullptr, 0, nullptr,
                                                            0, nullptr, M, N, K, alpha, beta, p.splits, p.kchunk, part,
-                                                           QknrArgs{}, sizeof(TO) == 4);
+                                                           QknrArgs{}, sizeof(TO) == 4 && p.parts);
           if (rc == KH_OK)
             gemm_splitk_reduce_kernel<TO><<<(int)(((int64_t)M * N / 4 + 255) / 256), 256, 0, stream()>>>(
                 part, p.splits, C, ldc, CI, ldcin, BI, M, N, alpha, beta);
@@ -1062,7 +1072,8 @@ int launch_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
         }
       }
       return launch_tile<TO, TA, USE_PLAIN>(choose_tile(sizeof(TA) == 4, M, N, K, 1), A, lda, (const uint16_t*)B, ldb, C,
-                                            ldc, CI, ldcin, BI, M, N, K, alpha, beta, 1, K, nullptr);
+                                            ldc, CI, ldcin, BI, M, N, K, alpha, beta, 1, K, nullptr, QknrArgs{},
+                                            p.parts);
     }
     if (trans_b && M == 1) {
       constexpr bool EX = std::is_same<TA, float>::value;
@@ -1211,6 +1222,7 @@ int kh_gemm_splitk_partials(const void* a, int64_t lda, const void* b, int64_t l
     p.splits = splits;
     p.kchunk = (((int)k + splits - 1) / splits + 127) / 128 * 128;
     p.tile = choose_tile(ab == 4, (int)m, (int)n, (int)k, splits);
+    p.parts = ab == 2 && narrow_split(m, n, (int)k, splits);
   }
   KH_REQUIRE(p.mfma && p.splits > 1 && p.splits == splits,
              "kh_gemm_splitk_partials: this product is not split %d ways (kh_gemm_split_count_for gives the count; "
@@ -1221,7 +1233,7 @@ int kh_gemm_splitk_partials(const void* a, int64_t lda, const void* b, int64_t l
                                                 part);
   return launch_tile<float, uint16_t, USE_SPLIT>(p.tile, (const uint16_t*)a, lda, (const uint16_t*)b, ldb, nullptr, 0,
                                                  nullptr, 0, nullptr, (int)m, (int)n, (int)k, 1.f, 0.f, p.splits,
-                                                 p.kchunk, part);
+                                                 p.kchunk, part, QknrArgs{}, p.parts);
 }
 
 int kh_gemm_swiglu(const void* x, int64_t ldx, const void* w_gu, int64_t ldw, void* h, int64_t ldh, int64_t m,

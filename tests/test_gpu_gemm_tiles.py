@@ -86,3 +86,20 @@ def test_bf16_products_sum_fp32_results_in_short_chains(hip, M, N, K):
     ref = x.astype(np.float64) @ w.astype(np.float64).T
     err = np.linalg.norm(y - ref) / np.linalg.norm(ref)
     assert err <= 1.1 * 2.0 ** -24 * np.sqrt(K / (16.0 * max(2, parts) * 6.0)), err
+
+
+@pytest.mark.parametrize("act", ["bfloat16", "float32"])
+@pytest.mark.parametrize("M,N,K", [(512, 1024, 640), (256, 1024, 640), (640, 512, 512), (200, 2048, 1016)])
+def test_short_sums_are_not_split(hip, act, M, N, K):
+    """Sums shorter than 1024 of more than a few tiles: one launch, and fp32 results of bf16 products still in short chains (a chain of
+    n steps is about 2^-24 sqrt(n / 6) of the result off; four of them, added at the end, half of one)."""
+    assert kernels.gemm_split_count(M, N, K, act) == 1
+    if act == "float32":
+        return
+    bits, x = syn.bf16(syn.normal(1, (M, K)))
+    wbits, w = syn.bf16(syn.normal(2, (N, K), 0.02))
+    y = F.dispatch_matmul(Tensor(bits, dtype="bfloat16"), Tensor(wbits, dtype="bfloat16"), transpose_b=True,
+                          out_dtype="float32").numpy().astype(np.float64)
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    err = np.linalg.norm(y - ref) / np.linalg.norm(ref)
+    assert err <= 0.7 * 2.0 ** -24 * np.sqrt(K / (16.0 * 6.0)), err
