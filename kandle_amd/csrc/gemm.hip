@@ -919,15 +919,19 @@ struct GemmPlan {
   bool parts = false;  // fp32 results of bf16 products are summed in PARTS
 };
 
-// Long fp32 sums of bf16 products whose 64 x 64 tiles leave CUs idle, split in fewer ways than would put
-// two such tiles on every CU, are taken in PARTS: the wider split can cost more than it gains (the
-// partials' way through memory), but its shorter chains are worth keeping.
+// The split that puts two 64 x 64 tiles on every CU (t64 of them unsplit, fewer than CUs); its k ranges.
+inline int wide_splits(int64_t t64, int K, int* kchunk) {
+  const int want = 2 * kCUs / t64 > kMaxSplits ? kMaxSplits : (int)(2 * kCUs / t64);
+  *kchunk = ((K + want - 1) / want + 127) / 128 * 128;
+  return (K + *kchunk - 1) / *kchunk;
+}
+// Long fp32 sums of bf16 products whose 64 x 64 tiles leave CUs idle, split in fewer ways than
+// wide_splits, are taken in PARTS: the wider split can cost more than it gains (the partials' way through
+// memory), but its shorter chains are worth keeping.
 inline bool narrow_split(int64_t M, int64_t N, int K, int splits) {
   const int64_t t64 = ((M + 63) / 64) * ((N + 63) / 64);
-  if (!(K >= 1024 && N % 4 == 0 && t64 < kCUs)) return false;
-  const int64_t want = 2 * kCUs / t64 > kMaxSplits ? kMaxSplits : 2 * kCUs / t64;
-  const int64_t kchunk = ((K + want - 1) / want + 127) / 128 * 128;
-  return splits < (K + kchunk - 1) / kchunk;
+  int kchunk;
+  return K >= 1024 && N % 4 == 0 && t64 > 0 && t64 < kCUs && splits < wide_splits(t64, K, &kchunk);
 }
 
 // aligned: both operands start on 16 bytes.  bf16: bf16 weights B with bf16 (a_bytes 2) or fp32
@@ -947,12 +951,18 @@ GemmPlan gemm_plan(bool aligned, int64_t lda, int64_t ldb, int M, int N, int K, 
   // (half the work per step) take the same split while 64 x 64 tiles fill less than five eighths of the
   // CUs, none from there on: 1000 x 1024 x 2048 split in two 10.1 us and 4.7 for the sum, unsplit 9.5;
   // 1500 x 1024 x 3072 18.5 and 11.4 against 18.6; 2000 x 2560 x 9728 102 and 22 against 125.
+  // From 6144 columns on five eighths to all of the CUs do better with two tiles each: 256 x 2560 x 9728 whole
+  // 43.6 us, in three (64 x 128 tiles) 29.7; 800 x 1024 x 9728 (208 tiles) 42.6 and 38.1; 150 x 5120 x 17408 (240)
+  // 73 and 63; 180 x 4096 x 6144 (192) 29.1 and 27.6; shorter sums go either way (256 x 2560 x 4096 20.8 and
+  // 16.8, 800 x 1024 x 4096 14.6 and 17.1) and stay whole.
   // Sums shorter than 1024 are split only while the tiles are few for their length: 512 x 1024 x 640 (128
   // tiles) bf16 split in two 8.2 us, whole 4.9, fp32 10.4 and 8.1; 128 x 1024 x 640 (32) bf16 6.6 and 4.7, fp32
   // 7.5 and 7.7; 300 x 1024 x 1000 (80) fp32 10.2 and 10.9.  (fp32 results of bf16 products keep the short
   // chains: 512 x 512 x 512 is 1.2e-7 off 64 bits in one chain, 6.3e-8 in PARTS.)
   const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
-  if (K >= 512 && N % 4 == 0 && (a_bytes == 4 || t64 < kCUs * 5 / 8)) {
+  if (a_bytes == 2 && K >= 6144 && N % 4 == 0 && t64 >= kCUs * 5 / 8 && t64 < kCUs) {
+    p.splits = wide_splits(t64, K, &p.kchunk);
+  } else if (K >= 512 && N % 4 == 0 && (a_bytes == 4 || t64 < kCUs * 5 / 8)) {
     float low = 0.f;
     for (int sp = 1; sp <= kMaxSplits; ++sp) {
       const int kchunk = ((K + sp - 1) / sp + 127) / 128 * 128;

@@ -103,3 +103,20 @@ def test_short_sums_are_not_split(hip, act, M, N, K):
     ref = x.astype(np.float64) @ w.astype(np.float64).T
     err = np.linalg.norm(y - ref) / np.linalg.norm(ref)
     assert err <= 0.7 * 2.0 ** -24 * np.sqrt(K / (16.0 * 6.0)), err
+
+
+@pytest.mark.parametrize("M,N,K,n", [(256, 2560, 9728, 3), (150, 5120, 6152, 2), (250, 2500, 6144, 3), (256, 2560, 4096, 1)])
+def test_long_bf16_sums_are_split(hip, M, N, K, n):
+    """bf16 products of five eighths to all of the CUs' 64 x 64 tiles: split from 6144 columns on.  The K
+    products are summed in fp32 (K 2^-24 sum |a w| at most), the bf16 result rounded (2^-8 of itself)."""
+    assert kernels.gemm_split_count(M, N, K) == n
+    assert kernels.gemm_split_count(M, 0, K) == 1
+    bits, x = syn.bf16(syn.normal(1, (M, K)))
+    wbits, w = syn.bf16(syn.normal(2, (N, K), 0.02))
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    ref, bar = x64 @ w64.T, K * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T)
+    for out in ("float32", "bfloat16"):
+        y = F.dispatch_matmul(Tensor(bits, dtype="bfloat16"), Tensor(wbits, dtype="bfloat16"), transpose_b=True,
+                              out_dtype=out).numpy().astype(np.float64)
+        most = bar if out == "float32" else bar + 2.0 ** -8 * (np.abs(ref) + bar)
+        assert np.all(np.abs(y - ref) <= most)
