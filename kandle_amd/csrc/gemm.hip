@@ -955,12 +955,14 @@ GemmPlan gemm_plan(bool aligned, int64_t lda, int64_t ldb, int M, int N, int K, 
   // 43.6 us, in three (64 x 128 tiles) 29.7; 800 x 1024 x 9728 (208 tiles) 42.6 and 38.1; 150 x 5120 x 17408 (240)
   // 73 and 63; 180 x 4096 x 6144 (192) 29.1 and 27.6; shorter sums go either way (256 x 2560 x 4096 20.8 and
   // 16.8, 800 x 1024 x 4096 14.6 and 17.1) and stay whole.
+  // So do a few fp32 rows, which stream weights: 9 x 2560 x 4096 in six 12.4 us, in eight 11.3.
   // Sums shorter than 1024 are split only while the tiles are few for their length: 512 x 1024 x 640 (128
   // tiles) bf16 split in two 8.2 us, whole 4.9, fp32 10.4 and 8.1; 128 x 1024 x 640 (32) bf16 6.6 and 4.7, fp32
   // 7.5 and 7.7; 300 x 1024 x 1000 (80) fp32 10.2 and 10.9.  (fp32 results of bf16 products keep the short
   // chains: 512 x 512 x 512 is 1.2e-7 off 64 bits in one chain, 6.3e-8 in PARTS.)
   const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
-  if (a_bytes == 2 && K >= 6144 && N % 4 == 0 && t64 >= kCUs * 5 / 8 && t64 < kCUs) {
+  const bool wide = a_bytes == 2 ? K >= 6144 && t64 >= kCUs * 5 / 8 : K >= 2048 && M <= 32;
+  if (wide && N % 4 == 0 && t64 > 0 && t64 < kCUs) {
     p.splits = wide_splits(t64, K, &p.kchunk);
   } else if (K >= 512 && N % 4 == 0 && (a_bytes == 4 || t64 < kCUs * 5 / 8)) {
     float low = 0.f;

@@ -120,3 +120,17 @@ def test_long_bf16_sums_are_split(hip, M, N, K, n):
                               out_dtype=out).numpy().astype(np.float64)
         most = bar if out == "float32" else bar + 2.0 ** -8 * (np.abs(ref) + bar)
         assert np.all(np.abs(y - ref) <= most)
+
+
+@pytest.mark.parametrize("M,N,K,n", [(9, 2560, 4096, 8), (32, 2560, 9728, 8), (9, 6144, 2568, 5), (9, 5120, 2048, 6),
+                                     (17, 100, 2056, 6)])
+def test_few_fp32_rows_are_split_widely(hip, M, N, K, n):
+    """Up to 32 fp32 rows, which stream weights: 512 / tiles parts of K, at most eight and of whole 128 columns.
+    Each product is 2^-16 off at most (the bf16 pair), the K of them are summed in fp32."""
+    assert kernels.gemm_split_count(M, N, K, "float32") == n
+    x = syn.normal(1, (M, K))
+    wbits, w = syn.bf16(syn.normal(2, (N, K), 0.02))
+    y = F.dispatch_matmul(Tensor(x), Tensor(wbits, dtype="bfloat16"), transpose_b=True).numpy().astype(np.float64)
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    bar = (2.0 ** -16 + K * 2.0 ** -24) * (np.abs(x64) @ np.abs(w64).T)
+    assert np.all(np.abs(y - x64 @ w64.T) <= bar)
