@@ -940,7 +940,7 @@ GemmPlan gemm_plan(bool aligned, int64_t lda, int64_t ldb, int M, int N, int K, 
                    int a_bytes, int min_rows) {
   GemmPlan p;
   const int64_t lim = int64_t(1) << 31;
-  if (!(bf16 && trans_b && M >= min_rows && K > 0 && K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned &&
+  if (!(bf16 && trans_b && M >= min_rows && K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned &&
         128 * lda * a_bytes < lim && 128 * ldb * 2 < lim))
     return p;
   p.mfma = true;

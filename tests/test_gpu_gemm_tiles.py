@@ -134,3 +134,15 @@ def test_few_fp32_rows_are_split_widely(hip, M, N, K, n):
     x64, w64 = x.astype(np.float64), w.astype(np.float64)
     bar = (2.0 ** -16 + K * 2.0 ** -24) * (np.abs(x64) @ np.abs(w64).T)
     assert np.all(np.abs(y - x64 @ w64.T) <= bar)
+
+
+@pytest.mark.parametrize("M", [9, 4194305])
+def test_no_columns(hip, M):
+    """K = 0: the C and bias terms alone, also for more rows than the generic kernel's grid holds."""
+    n = 8
+    c, b = Tensor(np.full((M, n), 3.0, np.float32)), Tensor(np.arange(n, dtype=np.float32))
+    a = Tensor(np.zeros((1, 8), np.uint16), dtype="bfloat16")
+    out = F.zeros((M, n))
+    kernels._lib.call("kh_gemm_ex", a.handle.data_ptr(), 0, 1, a.handle.data_ptr(), 0, 1, out.handle.data_ptr(), n,
+                      c.handle.data_ptr(), n, b.handle.data_ptr(), M, n, 0, 1.0, 0.5, 1, 0)
+    assert np.array_equal(out.numpy(), np.broadcast_to(1.5 + np.arange(n, dtype=np.float32), (M, n)))
