@@ -872,12 +872,14 @@ constexpr TileCost kTileBf16[kTiles] = {
 constexpr TileCost kTileF32[kTiles] = {
     {64, 64, .50f, 1.f}, {64, 128, .71f, 1.5f}, {128, 128, 1.19f, 2.f}, {128, 256, 1.75f, 3.f}, {256, 256, 3.2f, 5.f},
     {64, 192, .95f, 2.f}, {128, 192, 1.6f, 2.5f}};  // (not whole head rows: no QKNR)
-constexpr int kCUs = 256;
+// The compute units a plan fills: the device's, or an undivided card's before kh_init (the split count may be
+// asked for then).
+inline int cus() { return cu_count() > 0 ? cu_count() : 256; }
 
 inline float tile_cost(const TileCost& t, int64_t M, int64_t N, int64_t K, int splits) {
   const int64_t blocks = ((M + t.gm - 1) / t.gm) * ((N + t.gn - 1) / t.gn) * splits;
   const float steps = (float)((K + 63) / 64) / (float)splits;
-  return (float)((blocks + kCUs - 1) / kCUs) * (steps * t.step + t.ends);
+  return (float)((blocks + cus() - 1) / cus()) * (steps * t.step + t.ends);
 }
 // The tile of a product split `splits` ways; its cost in *cost if given.  heads: tiles of whole head rows.
 inline int choose_tile(bool f32, int M, int N, int K, int splits, bool heads = false, float* cost = nullptr) {
@@ -921,7 +923,7 @@ struct GemmPlan {
 
 // The split that puts two 64 x 64 tiles on every CU (t64 of them unsplit, fewer than CUs); its k ranges.
 inline int wide_splits(int64_t t64, int K, int* kchunk) {
-  const int want = 2 * kCUs / t64 > kMaxSplits ? kMaxSplits : (int)(2 * kCUs / t64);
+  const int want = 2 * cus() / t64 > kMaxSplits ? kMaxSplits : (int)(2 * cus() / t64);
   *kchunk = ((K + want - 1) / want + 127) / 128 * 128;
   return (K + *kchunk - 1) / *kchunk;
 }
@@ -931,7 +933,7 @@ inline int wide_splits(int64_t t64, int K, int* kchunk) {
 inline bool narrow_split(int64_t M, int64_t N, int K, int splits) {
   const int64_t t64 = ((M + 63) / 64) * ((N + 63) / 64);
   int kchunk;
-  return K >= 1024 && N % 4 == 0 && t64 > 0 && t64 < kCUs && splits < wide_splits(t64, K, &kchunk);
+  return K >= 1024 && N % 4 == 0 && t64 > 0 && t64 < cus() && splits < wide_splits(t64, K, &kchunk);
 }
 
 // aligned: both operands start on 16 bytes.  bf16: bf16 weights B with bf16 (a_bytes 2) or fp32
@@ -961,10 +963,10 @@ GemmPlan gemm_plan(bool aligned, int64_t lda, int64_t ldb, int M, int N, int K, 
   // 7.5 and 7.7; 300 x 1024 x 1000 (80) fp32 10.2 and 10.9.  (fp32 results of bf16 products keep the short
   // chains: 512 x 512 x 512 is 1.2e-7 off 64 bits in one chain, 6.3e-8 in PARTS.)
   const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
-  const bool wide = a_bytes == 2 ? K >= 6144 && t64 >= kCUs * 5 / 8 : K >= 2048 && M <= 32;
-  if (wide && N % 4 == 0 && t64 > 0 && t64 < kCUs) {
+  const bool wide = a_bytes == 2 ? K >= 6144 && t64 >= cus() * 5 / 8 : K >= 2048 && M <= 32;
+  if (wide && N % 4 == 0 && t64 > 0 && t64 < cus()) {
     p.splits = wide_splits(t64, K, &p.kchunk);
-  } else if (K >= 512 && N % 4 == 0 && (a_bytes == 4 || t64 < kCUs * 5 / 8)) {
+  } else if (K >= 512 && N % 4 == 0 && (a_bytes == 4 || t64 < cus() * 5 / 8)) {
     float low = 0.f;
     for (int sp = 1; sp <= kMaxSplits; ++sp) {
       const int kchunk = ((K + sp - 1) / sp + 127) / 128 * 128;
