@@ -1054,10 +1054,25 @@ int launch_prefill_d(const void* q, const void* k, const void* v, void* o, int b
   // Short calls: (32 queries x 32 keys) blocks per query head up to kDirectChunks in all.
   const int64_t nq32 = (lq + 31) / 32, nk32 = (lk + 31) / 32, full = nq32 < nk32 ? nq32 : nk32;
   const int64_t per_head = causal ? full * (full + 1) / 2 + (nq32 - full) * nk32 : nq32 * nk32;
-  if (per_head * batch * hq * D <= kDirectChunks * 128 && (causal || nq32 * batch * hq <= 448)) {
+  const int64_t blocks = nq32 * batch * hq, cu = cu_count();
+  // Items of the forms split over keys in two and in four (groups of up to four and up to two heads).
+  const int rows2 = G <= 4 ? 32 * (kPersistWaves / 2 / G) : 32, nqb2 = (lq + rows2 - 1) / rows2;
+  const int rows4 = G <= 2 ? 32 * (kPersistWaves / 4 / G) : 32, nqb4 = (lq + rows4 - 1) / rows4;
+  const int64_t items2 = (int64_t)nqb2 * batch * hkv, items4 = (int64_t)nqb4 * batch * hkv;
+  bool direct = per_head * batch * hq * D <= kDirectChunks * 128 && (causal || blocks <= 448);
+  // Where one whole tile of keys is all there is (97 to 128 queries, head dim 128), the forms below lose little
+  // to their staging once the CUs have several blocks each: 288 to 480 blocks 8.4 us there, 8.8 here (without
+  // the mask 7.8 and 8.8), 640 to 816 11.8-12.4 and 12.3-15.2; but 512 (where they split over keys) 11.6 and 9.1.
+  if (nq32 == 4 && D == 128 && G <= 4 && (blocks > 2 * cu || (G <= 2 && blocks > cu && items2 < cu / 2))) direct = false;
+  // Groups of four and eight heads read K and V once for all of them: 25 sequences of 32 with 64 / 8 heads 12.9
+  // us there, 15.5 here; 9 of 64 12.1 and 14.2 (head dim 64: 19 of 32 8.1 and 6.6, 16 of 64 9.2 and 10.8); 64 of
+  // 32 with 32 / 8 heads 16.6 and 17.8.
+  if ((G == 8 && blocks > (D == 64 && nq32 < 4 ? 5 : 4) * cu && nblk64 <= cu) || (G == 4 && D == 128 && blocks >= 8 * cu))
+    direct = false;
+  if (direct) {
     const Strides32 s32{(int32_t)st.qb, (int32_t)st.qh, (int32_t)st.qs, (int32_t)st.kb, (int32_t)st.kh, (int32_t)st.ks,
                         (int32_t)st.vb, (int32_t)st.vh, (int32_t)st.vs, (int32_t)st.ob, (int32_t)st.oh, (int32_t)st.os};
-    const int grid = (int)(nq32 * batch * hq), ratio = hq / hkv_real;
+    const int grid = (int)blocks, ratio = hq / hkv_real;
     const uint16_t *Q = (const uint16_t*)q, *K = (const uint16_t*)k, *V = (const uint16_t*)v;
     if (causal)
       flash_direct_kernel<true, D><<<grid, kDirectWaves * 64, 0, stream()>>>(Q, K, V, (uint16_t*)o, hq, ratio, lq, lk,
@@ -1074,36 +1089,31 @@ int launch_prefill_d(const void* q, const void* k, const void* v, void* o, int b
     // hold half the rows, when that gives at least half the CUs one (B = 1, 16 / 8 heads: S = 4096
     // 117.6 -> 103.0 us, 2048 63.4 -> 42.1, 1024 30.1 -> 24.6; shorter prompts keep the small
     // workgroups below).
-    // (groups of one or two query heads) a quarter of the rows, where that makes at most one and a half
-    // items per CU and more than one per two CUs: S = 1024 24.1 -> 21.0 us, 1531 31.0 -> 27.8; 2048 (two per CU) 38.5 either way, and
-    // two sequences of 1500 (three) 33 -> 49.
-    if (G <= 2) {
-      const int rows4 = 32 * (kPersistWaves / 4 / G), nqb4 = (lq + rows4 - 1) / rows4;
-      const int64_t items4 = (int64_t)nqb4 * batch * hkv;
-      if (2 * items4 > cu_count() && 2 * items4 <= 3 * cu_count()) {
-        persist(std::true_type{}, std::integral_constant<int, 4>{}, nqb4);
-        KH_CHECK_LAUNCH();
-        return KH_OK;
-      }
+    // (groups of one or two query heads, more than one tile of keys) a quarter of the rows, where that makes
+    // more than one item per two CUs and at most one per CU -- S = 1024 24.1 -> 21.0 us -- or up to one and a
+    // half, the more of them the longer the keys that pay for a CU's second: S = 1531 (384 items) 31.0 -> 27.8,
+    // two sequences of 600 (304) 18.7 -> 17.6; but four of 384 (384) 15.4 -> 18.1, one of 480 with 40 / 8 heads
+    // (320) 16.0 -> 17.7, two of 768 (384) 20.5 -> 21.2.  S = 2048 (two per CU) 38.5 either way, two sequences
+    // of 1500 (three) 33 -> 49.
+    const int64_t keys = lq < lk ? lq : lk;
+    if (G <= 2 && keys > 128 && 2 * items4 > cu && 2 * items4 <= 3 * cu &&
+        (items4 <= cu || keys >= 4 * (items4 - cu) + 11 * cu / 8)) {
+      persist(std::true_type{}, std::integral_constant<int, 4>{}, nqb4);
+      KH_CHECK_LAUNCH();
+      return KH_OK;
     }
-    const int BMQ2 = 32 * (kPersistWaves / 2 / G);
-    const int nqb2 = (lq + BMQ2 - 1) / BMQ2;
-    if ((int64_t)nqb2 * batch * hkv >= cu_count() / 2) {
+    if (items2 >= cu / 2) {
       persist(std::true_type{}, std::integral_constant<int, 2>{}, nqb2);
       KH_CHECK_LAUNCH();
       return KH_OK;
     }
   }
-  if (!causal && G <= 4 && nblk64 < kSmallGrid && lk > 256) {
+  if (!causal && G <= 4 && nblk64 < kSmallGrid && lk > (G == 4 && items2 <= cu ? 320 : 256)) {
     // Few equal items: the key-split form with the fewest tile times (one of the form split in two takes
     // about 1.2 of those of the form split in four, for twice the rows), if the items fill half the chip
     // and have a few tiles to share out.  16 / 8 heads, against the workgroups below: one sequence of 1024
     // 29.1 -> 22.1 us, 1531 79.2 -> 32.4, 2600 193 -> 92; four of 300 25.4 -> 15.1; eight of 128 (one tile)
-    // 8.8 there, 10.8 here.
-    const int rows2 = 32 * (kPersistWaves / 2 / G), nqb2 = (lq + rows2 - 1) / rows2;
-    const int64_t cu = cu_count(), items2 = (int64_t)nqb2 * batch * hkv;
-    const int rows4 = G <= 2 ? 32 * (kPersistWaves / 4 / G) : rows2, nqb4 = (lq + rows4 - 1) / rows4;
-    const int64_t items4 = (int64_t)nqb4 * batch * hkv;
+    // 8.8 there, 10.8 here; two of 320 with 32 / 8 heads 13.9 there, 14.5 here.
     if (G <= 2 && items4 >= cu / 2 && 5 * ((items4 + cu - 1) / cu) <= 6 * ((items2 + cu - 1) / cu)) {
       persist(std::false_type{}, std::integral_constant<int, 4>{}, nqb4);
       KH_CHECK_LAUNCH();

@@ -71,3 +71,16 @@ def test_direct_kernel_strided_views(hip):
 def test_key_split_forms(hip, B, hq, hkv, lq, lk, d, causal):
     rows = [0, 1, 31, 32, 63, 64, 127, 128, lq // 2, lq - 33, lq - 2, lq - 1]
     _check(B, hq, hkv, lq, lk, d, causal, rows=rows)
+
+
+# Both sides of the limits between the kernel without shared tiles, the forms split over keys and the small
+# workgroups: 97 to 128 queries of more than one block per CU, and of exactly two; groups of eight and four heads
+# of many short sequences; items split in four up to one per CU and beyond it with few and enough keys; groups
+# of four without the mask.
+@pytest.mark.parametrize("B,hq,hkv,S,d,causal", [
+    (4, 16, 8, 128, 128, True), (5, 16, 8, 127, 128, True), (8, 16, 8, 128, 128, True), (9, 16, 8, 128, 128, True),
+    (5, 16, 8, 126, 128, False), (16, 64, 8, 32, 128, True), (17, 64, 8, 31, 128, True), (64, 32, 8, 30, 128, True),
+    (2, 16, 8, 512, 64, True), (4, 16, 8, 384, 128, True), (2, 16, 8, 600, 128, True), (3, 16, 8, 420, 64, True),
+    (1, 40, 8, 480, 128, True), (2, 32, 8, 320, 128, False), (2, 32, 8, 321, 64, False)])
+def test_forms_beside_their_limits(hip, B, hq, hkv, S, d, causal):
+    _check(B, hq, hkv, S, S, d, causal, rows=sorted({0, 1, 31, min(32, S - 1), S // 2, S - 2, S - 1}))
