@@ -83,4 +83,4 @@ def test_key_split_forms(hip, B, hq, hkv, lq, lk, d, causal):
     (2, 16, 8, 512, 64, True), (4, 16, 8, 384, 128, True), (2, 16, 8, 600, 128, True), (3, 16, 8, 420, 64, True),
     (1, 40, 8, 480, 128, True), (2, 32, 8, 320, 128, False), (2, 32, 8, 321, 64, False)])
 def test_forms_beside_their_limits(hip, B, hq, hkv, S, d, causal):
-    _check(B, hq, hkv, S, S, d, causal, rows=sorted({0, 1, 31, min(32, S - 1), S // 2, S - 2, S - 1}))
+    _check(B, hq, hkv, S, S, d, causal, rows=sorted({0, 1, min(32, S - 1), S // 2, S - 2, S - 1}))
