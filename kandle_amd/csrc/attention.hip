@@ -692,8 +692,38 @@ __device__ __forceinline__ void decode_merge_cols_body(const float* __restrict__
       lc[u] = mlc.y;
       oc[u] = po[(int64_t)cc * D];
     }
+    if constexpr (SH > 1) {
+      // Quarter chunks are four times as many: weighted by the pass's maximum and added pairwise, so that
+      // their chains of fp32 additions are no longer than the full chunks' (one fp32 sequence of 6000 keys,
+      // 188 chunks: 2.03e-7 against 64 bits one after another, 1.87e-7 this way, 1.95e-7 with 47 full chunks).
+      float mb = m;
 #pragma unroll
-    for (int u = 0; u < U; ++u) fold(c + u * NG < nch ? mc[u] : -INFINITY, lc[u], oc[u]);
+      for (int u = 0; u < U; ++u) {
+        if (c + u * NG >= nch) mc[u] = -INFINITY;
+        mb = fmaxf(mb, mc[u]);
+      }
+      const float mu = mb == -INFINITY ? 0.f : mb;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float p = __expf(mc[u] - mu);
+        lc[u] *= p;
+        oc[u] *= p;
+      }
+#pragma unroll
+      for (int s = 1; s < U; s *= 2)
+#pragma unroll
+        for (int u = 0; u < U; u += 2 * s) {
+          lc[u] += lc[u + s];
+          oc[u] += oc[u + s];
+        }
+      const float a = __expf(m - mu);
+      l = l * a + lc[0];
+      acc = acc * a + oc[0];
+      m = mb;
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u) fold(c + u * NG < nch ? mc[u] : -INFINITY, lc[u], oc[u]);
+    }
   }
   if (col == 0) {
     gm[grp] = m;
