@@ -336,6 +336,8 @@ int kh_flash_attention_masked(const void* q, const void* k, const void* v, void*
  * (strides: batch, head, seq).  `strides` holds 10 values: q (b, h), k (b, h, s), v (b, h, s),
  * o (b, h).  Split-K over the sequence with a log-sum-exp merge; bf16 or f32; d == 64 or 128;
  * any GQA ratio; q and the caches 16-byte aligned with strides in 16-byte units.
+ * The chunk size of the split follows batch, heads and max_len, so a sequence's output can differ in
+ * its last bits with the batch that it is part of and the cache that holds it.
  * Varlen extension of flash_attention for StaticKVCache views
  * (reference: packages/model-utils/src/kv-cache.ts:197-211; register.ts:102-109). */
 int kh_decode_attention(const void* q, const void* k_cache, const void* v_cache, void* o,

@@ -804,14 +804,25 @@ inline int decode_group_heads(int G) {
 // kernels of a call, head dim 128, 16 / 8 heads, full -> quarter chunks: two fp32 sequences of 777 keys
 // 11.5 -> 7.7 us, seven of 1280 17.0 -> 14.5; one bf16 of 600 8.4 -> 6.8, eight of 2100 (9 chunks each)
 // 16.0 -> 13.2; on the other side five bf16 of 3000 (480 chunks, 12 each) 13.2 -> 13.5, one fp32 of 16000
-// 23.8 -> 28.3.  (The quarter chunks' partials stay within the allocation-free entry's scratch.)
+// 23.8 -> 28.3.  Full chunks that fill every CU the same number of times leave nothing to spread: sixteen
+// bf16 sequences of 512 with 16 / 16 heads (512 chunks) 11.2 -> 13.8, of 1000 with 32 / 8 (512) 18.3 -> 21.2; eight
+// or fewer sequences go either way there and take quarters (eight of 1000 with 16 / 8 heads, 256 chunks, 10.5 ->
+// 9.5, with 40 / 8 14.7 -> 15.8), but not where seven or eight heads share a chunk, whose waves are bound by
+// their arithmetic (one of 8000 with 64 / 8 heads 18.0 -> 20.7).  fp32 pairs of heads gain there too (16 / 8
+// heads, sixteen of 512 15.7 -> 14.3).  (The quarter chunks' partials stay within the allocation-free entry's
+// scratch.)
 template <typename T, int DH>
 inline int decode_shrink(int batch, int hq, int hkv, int64_t max_len) {
   constexpr int CH = dc_chunk<T, DH>(), small = dc_chunk<T, DH, 4>();
   const int64_t per_seq = (max_len + CH - 1) / CH;
-  const int64_t chunks = per_seq * (hq / decode_group_heads(hq / hkv)) * batch;
+  const int heads = decode_group_heads(hq / hkv);
+  const int64_t chunks = per_seq * (hq / heads) * batch;
   const bool f32 = sizeof(T) == 4;
   if (!(chunks < (f32 ? 512 : 400) || (chunks < 1200 && per_seq <= (f32 ? 17 : 9)))) return 1;
+  const int64_t cu = cu_count(), rounds = (chunks + cu - 1) / cu;
+  const bool whole = 4 * (per_seq * CH - max_len) < CH;  // the longest sequence's last chunk is a whole one, nearly
+  if (batch > 8 && chunks == rounds * cu && whole && !(f32 && heads == 2)) return 1;
+  if (heads >= 7 && 8 * chunks >= 7 * rounds * cu && (whole || per_seq >= 8)) return 1;
   const int64_t bytes = (int64_t)batch * hq * ((max_len + small - 1) / small) * (DH + 2) * (int64_t)sizeof(float);
   return bytes <= (int64_t)kNoAllocScratchBytes ? 4 : 1;
 }

@@ -73,3 +73,21 @@ def test_quarter_chunks_are_as_exact_as_full_chunks(hip, hq, hkv, L):
             got = F.decode_attention(Tensor(q), kc, vc, sl, scale).numpy()[0].astype(np.float64)
             err[i] += np.linalg.norm(got - ref) / np.linalg.norm(ref)
     assert err[0] <= 1.01 * err[1], err / 4
+
+
+@pytest.mark.parametrize("dtype,B,hq,hkv,L,d", [
+    ("bfloat16", 16, 16, 16, 512, 128), ("bfloat16", 16, 16, 16, 440, 128), ("float32", 16, 16, 8, 256, 128),
+    ("bfloat16", 8, 64, 8, 1000, 128), ("bfloat16", 1, 64, 8, 8000, 128), ("float32", 1, 64, 8, 6000, 128)])
+def test_both_sides_of_whole_rounds(hip, dtype, B, hq, hkv, L, d):
+    """Caches whose full chunks fill the CUs a whole number of times, which keep full chunks for more than
+    eight sequences and for groups of eight heads, and those beside them: against the oracle."""
+    q, qh = _case(1, (B, hq, d), dtype)
+    k, kh = _case(2, (B, hkv, L, d), dtype)
+    v, vh = _case(3, (B, hkv, L, d), dtype)
+    lens = np.linspace(L // 4, L, B).astype(np.int32)
+    scale = 1.0 / np.sqrt(d)
+    got = F.decode_attention(q, k, v, Tensor(lens, dtype="int32"), scale).numpy()
+    for b in {0, B // 2, B - 1}:
+        n = lens[b]
+        ref = oracle.sdpa(qh[b][None, :, None], kh[b][None, :, :n], vh[b][None, :, :n], scale=scale)[0, :, 0]
+        assert np.abs(got[b] - ref).max() <= np.abs(ref).max() * (1e-4 if dtype == "float32" else 2.0 ** -7)
