@@ -1,10 +1,12 @@
 // bf16 causal / non-causal GQA flash-attention prefill for gfx950, head_dim 64 or 128, and the
 // split-bf16 fp32 attention of the float32-activation model.
 //
-// Launch forms of the bf16 kernel (launch_prefill_d): the tile kernel (one workgroup per query
-// block, 8 waves, or 2-4 waves on small grids); the persistent form for causal inputs with at least
-// two 128-row items per CU (C3); its key-split form for one or two long sequences (too few items to
-// pair); GQA ratios other than 1, 2, 4, 8 as groups of query heads on all of them.
+// Launch forms of the bf16 kernel (launch_prefill_d): the kernel without shared tiles for short calls
+// (flash_direct_kernel); the tile kernel (one workgroup per query block, 8 waves, or 2-4 waves on small
+// grids); the persistent form for causal inputs with at least two 128-row items per CU (C3); its key-split
+// forms, the keys of a row shared by two or four waves, for causal calls with too few items to pair (one or
+// two long sequences) and for few items without the mask; GQA ratios other than 1, 2, 4, 8 as groups of
+// query heads on all of them.
 //
 // Semantics follow the reference kernel (packages/backend-webgpu/src/kernels/attention/builder.ts:138-329):
 // score = (q . k) * scale, key j > query i masked when causal (top-left), query head h reads kv head
@@ -13,7 +15,8 @@
 // A workgroup of WAVES waves shares one kv head: wave w serves query head g = w / (WAVES/G) of the
 // G query heads that read this kv head (G = hq / hkv <= WAVES) and 32 query rows of a
 // BMQ = 32 * WAVES / G row block.  K/V tiles of BN keys (128) are staged in LDS (double buffered, one
-// barrier per tile) and shared by all waves, which compute them in chunks of 64 keys.
+// barrier per tile) and shared by all waves, which compute them in chunks of 64 keys (32 where four
+// waves share a row's keys).
 //
 // Per wave and chunk, with v_mfma_f32_32x32x16_bf16:
 //   S^T (keys x queries) = K Q^T : A = K rows from LDS, B = Q held in registers for the whole loop.
@@ -830,14 +833,17 @@ constexpr int kSmallBN = 128;
 // Short calls are bound by latency: the tile kernels load, store to LDS, cross a barrier and read back
 // for every 128 keys, and a few dozen query blocks leave most CUs idle; here a block's chain is a
 // quarter of its 32-key chunks and no wave waits for another.  Each wave reads its own K and V from L2,
-// though (16 KiB per chunk at head dim 128, about 9.5 TB/s over the chip), which bounds longer calls:
+// though (16 KiB per chunk at head dim 128: 44 MB in the 9.4 us of 480 tokens), which bounds longer calls:
 // hence the limit on the number of chunks.  One sequence, 16 / 8 heads, head dim 128, causal, against the
 // forms below: S = 64 7.5 -> 5.8 us, 256 11.5 -> 8.0, 480 16.9 -> 10.5; S = 1024 24.2 -> 27.5 (8448 chunks).
-// The limit of 2048 chunks keeps 512-token prompts of 16 heads (2176 chunks, 17.7 -> 10.9) on the forms
-// below: their sums decide the bf16 model's logits to the last few percent of the tolerance its parity
-// test allows, and either grouping of the chunks here was over it (0.0201 and 0.0203 of 0.02; 0.0194
-// there).  Without the causal mask the chains are equal and short calls of many
-// blocks stay on the tile kernels (eight sequences of 128, 512 blocks: 8.7 us there, 9.5 here).
+// It is also the more exact one: error against 64 bits 0.97 of the forms below at the same inputs.  By time the
+// limit could lie higher (512 tokens of 16 heads, 2176 chunks, 17.7 -> 10.9 us; the crossing is at some 7000).
+// It stays under those because any other grouping of their chunks moves the bf16 model's logits by other
+// roundings -- as far from its oracle in 2-norm, 5.0e-3 to 6.6e-3 over three models and 200 to 512 tokens with
+// either form, but the largest difference of one 512-token generation is held to 0.02 and comes to 0.0194
+// with the forms below, 0.0201 and 0.0203 with two groupings of this one.  Without the causal mask the chains
+// are equal and short calls of many blocks stay on the tile kernels (eight sequences of 128, 512 blocks: 8.7
+// us there, 9.5 here); launch_prefill_d names the other shapes that do.
 constexpr int kDirectWaves = 4;
 constexpr int64_t kDirectChunks = 2048;
 using FL128 = Flash<128, 8, 128>;  // for its swap23 and 32-bit strides

@@ -1,8 +1,11 @@
 // GEMM for the projections: C = alpha * A * B' + beta * Cin (+ bias), fp32 accumulate.
 //
-//  * bf16 inputs, trans_b = 1 (nn.Linear weight [n, k]), m > 8: MFMA tile kernel
-//    (v_mfma_f32_32x32x16_bf16).
-//  * m <= 8, trans_b = 1: weight-streaming kernel that reads each weight row once (decode, lm_head).
+//  * bf16 weights, trans_b = 1 (nn.Linear weight [n, k]), m > 8: MFMA tile kernel
+//    (v_mfma_f32_32x32x16_bf16); so are most bf16 products of two to eight rows (tile_min_rows: all with bf16
+//    results but two short rows against few columns, and those with fp32 results whose rows do not fit LDS).
+//  * bf16 weights, m = 1: one-row kernel that reads each weight row once (decode, lm_head); fp32 rows, two to
+//    eight, too long for LDS go through it one by one.
+//  * otherwise m <= 8, trans_b = 1: skinny kernel, the rows in LDS as fp32.
 //  * anything else: LDS-tiled fp32-math kernel.
 // The output (and Cin / bias) may be bf16 or fp32 independently of bf16 inputs, e.g. fp32 logits.
 //
@@ -305,7 +308,7 @@ __device__ __forceinline__ void gemm_wave_store(const f32x16 (&acc)[AN][AM], cha
 // up to five of them are in flight, and there is one barrier per stage.  A wave's copy writes 1 KiB of
 // consecutive LDS bytes, so rows are stored without padding and the 16-byte chunks of a row are permuted
 // instead (chunk c of row i at place c ^ swz(i)): the 16 lanes that one cycle of a fragment read serves
-// then fall on 16 different bank groups (no bank conflicts counted).  Measured against the register-staged
+// then fall on 16 different bank groups (no bank conflicts counted in the k loop).  Measured against the register-staged
 // kernel before it (two LDS buffers, 64 x 64 to 128 x 128 tiles), one call, weights from HBM:
 //   bf16  512 x 4096 x 1024  13.0 ->  9.4 us     fp32  512 x 4096 x 1024  19.3 -> 14.8 us
 //   bf16 1000 x 4096 x 1024  19.9 -> 14.4 us     fp32 1000 x 4096 x 1024  30.4 -> 23.1 us
@@ -619,7 +622,8 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
 }
 
 // =============================================================================================
-// Skinny kernel for m <= 8 (trans_b = 1): each wave owns output columns n and streams weight row n
+// Skinny kernel for m <= 8 (trans_b = 1, rows that fit 64 KiB of LDS; bf16 ones mostly take the tiles,
+// tile_min_rows): each wave owns output columns n and streams weight row n
 // once with 16-byte loads; the m rows of A are kept in LDS as fp32.
 // =============================================================================================
 constexpr int SK_MAXM = 8;
