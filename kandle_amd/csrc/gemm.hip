@@ -910,7 +910,7 @@ inline bool fits_skinny(int64_t M, int64_t K) { return M <= SK_MAXM && M * K * (
 // columns stay (2 x 4096 x 1024: 11.0 there, 12.3 on tiles).  fp32 results keep the
 // skinny kernel's 64-way sums (error against 64 bits 7e-8 at K = 1024, the tiles' 8e-8) as long as its rows
 // fit LDS; beyond, the generic kernel's one sum over K (1e-6 at K = 9728) was both slower and less
-// exact: bf16 rows take the tiles there (8 x 2560 x 9728 1529 -> 13.9 us, error 2.5e-7), fp32 rows the
+// exact: bf16 rows take the tiles there (8 x 2560 x 9728 1529 -> 13.9 us, error 1.3e-7), fp32 rows the
 // one-row kernel row by row (1542 -> 141 us, 2.3e-7; its exact products, which the tiles' split of
 // fp32 rows into two bf16 would not keep).
 inline int tile_min_rows(int a_bytes, int out_bytes, int M, int N, int K) {

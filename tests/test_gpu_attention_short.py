@@ -84,3 +84,14 @@ def test_key_split_forms(hip, B, hq, hkv, lq, lk, d, causal):
     (1, 40, 8, 480, 128, True), (2, 32, 8, 320, 128, False), (2, 32, 8, 321, 64, False)])
 def test_forms_beside_their_limits(hip, B, hq, hkv, S, d, causal):
     _check(B, hq, hkv, S, S, d, causal, rows=sorted({0, 1, min(32, S - 1), S // 2, S - 2, S - 1}))
+
+
+@pytest.mark.parametrize("B,hq,hkv,S,d,causal", [
+    (1, 16, 8, 1531, 128, True), (1, 16, 8, 300, 128, True), (2, 16, 8, 600, 64, True), (1, 16, 8, 1000, 128, False),
+    (1, 32, 8, 700, 128, False)])
+def test_forms_repeat_themselves(hip, B, hq, hkv, S, d, causal):
+    """The same call gives the same bits every time: the parts of the keys are merged in a fixed order."""
+    q, k, v = (_bf(s, (B, h, S, d))[0] for s, h in ((1, hq), (2, hkv), (3, hkv)))
+    first = F.scaled_dot_product_attention(q, k, v, is_causal=causal).numpy()
+    for _ in range(4):
+        assert np.array_equal(F.scaled_dot_product_attention(q, k, v, is_causal=causal).numpy(), first)
